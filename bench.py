@@ -315,7 +315,7 @@ def producer_bench(args, torch, stream):
                               f"attn_fwd_bf16_kernel intra-frame, {frames} frames, "
                               f"{att_flops} flop"),
             "out_proj": roof("mfma", out_flops, out_ms, BF16_PEAK_TFLOPS, "TFLOP/s",
-                             f"proj_gemm_bf16_small_kernel, 1 group, fp32 residual added in the epilogue, {out_flops} flop"),
+                             f"proj_gemm_small_kernel, 1 group, fp32 residual added in the epilogue, {out_flops} flop"),
         },
     }
     if not args.no_cpu_baseline:

@@ -110,16 +110,17 @@ int layer_stage_launch(void* stager, void* arena, const void* k, const void* v, 
 // n 32-bit words at dst set to value, on the stream (a kernel, no memset node).
 int fill_words(void* dst, long n, unsigned value, void* stream);
 
-// Grouped bf16 projection GEMM (proj_gemm.hip): for g < groups (1..3),
+// Grouped projection GEMM (proj_gemm.hip): for g < groups (1..3),
 // outs[g][r, n] = sum_k x[r, k] w[g*Ng + n, k] + bias[g*Ng + n]
-// (+ outs[g][r, n] when accumulate; fp32 output only). x, w bf16; bias fp32
-// or null; out_dtype 0 = fp32, 1 = bf16; tile_n 128 (128 x 128 tiles, two
-// workgroups per CU) or 256 (256 x 256 tiles, one workgroup per CU).
-// Returns 0 on success, 2 when the shape is outside the
-// kernel's tiling (K % 64 or Ng % tile_n), 1 on any other error.
-int launch_proj_gemm(const void* x, const void* w, const float* bias, void* const* outs,
-                     int groups, long rows, int K, int Ng, int out_dtype, bool accumulate,
-                     int tile_n, void* stream);
+// (+ outs[g][r, n] when accumulate; fp32 output only). x, w of in_dtype (0 =
+// fp32, 1 = bf16); bias fp32 or null; out_dtype 0 = fp32, 1 = bf16 (fp32
+// operands: fp32 only); tile_n 128 (128 x 128 tiles, two workgroups per CU)
+// or 256 (bf16 operands: 256 x 256 tiles, one workgroup per CU).
+// Returns 0 on success, 2 when the shape is outside the kernel's tiling
+// (K % 64, fp32 K % 32, or Ng % tile_n), 1 on any other error.
+int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bias,
+                     void* const* outs, int groups, long rows, int K, int Ng, int out_dtype,
+                     bool accumulate, int tile_n, void* stream);
 // Any-shape linear layer (proj_gemm.hip, fp32 matrix cores):
 // y[r, n] = sum_k x[r, k] w[n, k] + bias[n] (+ y[r, n] when accumulate, fp32
 // output only); in/out dtype pairs fp32->fp32, bf16->bf16, bf16->fp32.

@@ -1,10 +1,11 @@
-// Grouped bf16 projection GEMM for the K/V producer, gfx950 (CDNA4).
+// Grouped projection GEMM for the K/V producer, gfx950 (CDNA4).
 //
 //   out_g[r, n] = sum_k x[r, k] * w[g*Ng + n, k] + bias[g*Ng + n]  (+ out_g[r, n])
 //
-// for groups g < G, with x [rows, K] and w [G*Ng, K] bf16 row-major (both
-// K-contiguous), bias fp32, out_g [rows, Ng] bf16 or fp32 (fp32 may
-// accumulate into itself: the residual add of out_proj). One launch covers
+// for groups g < G, with x [rows, K] and w [G*Ng, K] bf16 or fp32 row-major
+// (both K-contiguous), bias fp32, out_g [rows, Ng] bf16 or fp32 (fp32 may
+// accumulate into itself: the residual add of out_proj; fp32 operands give
+// fp32 outputs). One launch covers
 // every group, so the three q/k/v projections of a DiT block
 // (reference: src/backbone.py:13,18-19) run as one grid written straight to
 // three token-major outputs, and out_proj (src/backbone.py:22,32-33) adds
@@ -13,7 +14,8 @@
 // Two tilings share the operand layout below: the large-tile kernel (256 x
 // 256, one workgroup per CU) and the small-tile kernel (128 x 128, two
 // workgroups per CU, described at its definition), which is the faster one
-// at the backbone's shapes and the one the q/k/v projection uses.
+// at the backbone's shapes and the one the q/k/v projection uses. fp32 operands
+// always take the small tiles.
 //
 // Work decomposition (large tiles):
 //   workgroup = 4 waves, output tile TN features x 256 tokens; wave (wn, wr)
@@ -41,8 +43,8 @@
 //   few token tiles and a run of weight tiles through its L2.
 //
 // Token rows past `rows` read as zeros (buffer bounds) and are not stored.
-// Requirements (checked on the host): K % 64 == 0, Ng % TN == 0, 16-byte
-// aligned operands.
+// Requirements (checked on the host): K % 64 == 0 (fp32 operands: K % 32),
+// Ng % TN == 0, 16-byte aligned operands.
 
 #include <hip/hip_runtime.h>
 
@@ -67,8 +69,8 @@ constexpr int kPNumXcd = 8;
 constexpr int kPBufFlags = 0x00020000;
 
 struct ProjArgs {
-    const __bf16* x;
-    const __bf16* w;
+    const void* x;
+    const void* w;
     const float* bias;
     void* out[3];
     long rows;
@@ -149,8 +151,8 @@ __global__ __launch_bounds__(kPThreads, 1) void proj_gemm_bf16_kernel(ProjArgs a
 
     // ---- copy setup: instruction i of a wave fills 1 KiB = 8 rows ----
     const unsigned kbytes = (unsigned)a.K * 2u;
-    const __bf16* wg_base = a.w + ((long)g * a.Ng + n0) * a.K;
-    const __bf16* xg_base = a.x + r0 * a.K;
+    const __bf16* wg_base = static_cast<const __bf16*>(a.w) + ((long)g * a.Ng + n0) * a.K;
+    const __bf16* xg_base = static_cast<const __bf16*>(a.x) + r0 * a.K;
     long xrows = a.rows - r0;
     if (xrows > kPTileR) xrows = kPTileR;
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
@@ -354,8 +356,22 @@ __global__ __launch_bounds__(kPThreads, 1) void proj_gemm_bf16_kernel(ProjArgs a
 // after the barrier that frees their stage. With two resident workgroups the
 // one in its epilogue or waiting on copies leaves the MFMA pipe to the other,
 // and four times as many tiles even out the rounds over the CUs.
-template <int TN, int TR, typename OutT, bool kAcc>
-__global__ __launch_bounds__(kPThreads, 2) void proj_gemm_bf16_small_kernel(ProjArgs a) {
+//
+// InT is the operands' type. A stage row is 128 bytes of K either way (64 bf16
+// or 32 fp32 values), so copies, swizzle and fragment reads are the same
+// bytes; a 16-byte fragment holds 8 bf16 values of k (one
+// v_mfma_f32_32x32x16_bf16) or 4 fp32 ones (four v_mfma_f32_32x32x2_f32, each
+// pairing value e of the lower half-wave's fragment with value e of the upper
+// one's, in both operands alike).
+//
+// fp32 (q/k/v of one frame, 1560 rows, K = 1536, 3 x 1536 features) is bound by
+// the fp32 matrix cores (157 TFLOP/s peak): LayerNorm and this launch take
+// 187 us, 123 TFLOP/s in the GEMM; three launches of the bounds-checked
+// any-shape kernel below took 696 us with the same LayerNorm. A chunk's 64
+// MFMAs per wave (4,096 cycles) cover its copies many times over. 468
+// workgroups on 512 slots leave 9 % of the chip idle.
+template <typename InT, int TN, int TR, typename OutT, bool kAcc>
+__global__ __launch_bounds__(kPThreads, 2) void proj_gemm_small_kernel(ProjArgs a) {
     constexpr int JN = TN / 64, JR = TR / 64;
     constexpr int kWB = TN * kPRowBytes, kXB = TR * kPRowBytes, kSB = kWB + kXB;
     constexpr int kWC = kWB / 4096, kXC = kXB / 4096, kCP = kWC + kXC;  // copies per wave
@@ -383,14 +399,15 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_bf16_small_kernel(Proj
     const int wn = wave & 1;
     const int wr = wave >> 1;
 
-    const unsigned kbytes = (unsigned)a.K * 2u;
+    const unsigned kbytes = (unsigned)a.K * (unsigned)sizeof(InT);
     long xrows = a.rows - r0;
     if (xrows > TR) xrows = TR;
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<__bf16*>(a.w + ((long)g * a.Ng + n0) * a.K), (short)0, (int)(TN * kbytes),
-        kPBufFlags);
+        const_cast<InT*>(static_cast<const InT*>(a.w) + ((long)g * a.Ng + n0) * a.K), (short)0,
+        (int)(TN * kbytes), kPBufFlags);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<__bf16*>(a.x + r0 * a.K), (short)0, (int)(xrows * (long)kbytes), kPBufFlags);
+        const_cast<InT*>(static_cast<const InT*>(a.x) + r0 * a.K), (short)0,
+        (int)(xrows * (long)kbytes), kPBufFlags);
     const unsigned lds0 = (unsigned)(uintptr_t)lds;
     // copy c of a chunk: 1 KiB block blk of the weight (c < kWC) or token
     // operand, rows 8*blk + lane/8, physical chunk lane % 8
@@ -441,7 +458,7 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_bf16_small_kernel(Proj
         }
     }
 
-    const int nk = a.K / kPChunkK;
+    const int nk = (int)(kbytes / kPRowBytes);
     constexpr int kFeat = TN / 2;
     constexpr int kEs = (int)sizeof(OutT);
     constexpr int kChunks = kFeat * kEs / 16;
@@ -503,13 +520,25 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_bf16_small_kernel(Proj
             pj_lgkm_wait(cur);
             if (ks < 3) read_frags(fr[(ks + 1) & 1], st, ks + 1);
             __builtin_amdgcn_s_setprio(1);
+            if constexpr (sizeof(InT) == 2) {
 #pragma unroll
-            for (int i = 0; i < JN; ++i)
+                for (int i = 0; i < JN; ++i)
 #pragma unroll
-                for (int j = 0; j < JR; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, cur[i]), __builtin_bit_cast(bf16x8, cur[JN + j]),
-                        acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < JR; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, cur[i]),
+                            __builtin_bit_cast(bf16x8, cur[JN + j]), acc[i][j], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < JN; ++i)
+#pragma unroll
+                        for (int j = 0; j < JR; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                __uint_as_float(cur[i][e]), __uint_as_float(cur[JN + j][e]),
+                                acc[i][j], 0, 0, 0);
+            }
             __builtin_amdgcn_s_setprio(0);
         }
     }
@@ -577,16 +606,16 @@ void launch_large(const ProjArgs& a, hipStream_t st) {
                        dim3(kPThreads), 0, st, a);
 }
 
-template <typename OutT, bool kAcc>
+template <typename InT, typename OutT, bool kAcc>
 void launch_small(const ProjArgs& a, hipStream_t st) {
     const int grid = a.n_tiles * a.r_tiles;
-    hipLaunchKernelGGL((proj_gemm_bf16_small_kernel<kPSmall, kPSmall, OutT, kAcc>),
+    hipLaunchKernelGGL((proj_gemm_small_kernel<InT, kPSmall, kPSmall, OutT, kAcc>),
                        dim3((unsigned)grid), dim3(kPThreads), 0, st, a);
 }
 
 
 // ---------------------------------------------------------------------------
-// Generic linear layer (shapes the grouped kernel does not tile, and fp32):
+// Generic linear layer (shapes and alignments the grouped kernel does not take):
 //
 //   y[r, n] = sum_k x[r, k] * w[n, k] + bias[n]  (+ y[r, n])
 //
@@ -790,12 +819,9 @@ int launch_gemm_generic(int in_dtype, int out_dtype, const void* x, const void* 
     return 0;
 }
 
-namespace {
-}  // namespace
-
-int launch_proj_gemm(const void* x, const void* w, const float* bias, void* const* outs,
-                     int groups, long rows, int K, int Ng, int out_dtype, bool accumulate,
-                     int tile_n, void* stream) {
+int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bias,
+                     void* const* outs, int groups, long rows, int K, int Ng, int out_dtype,
+                     bool accumulate, int tile_n, void* stream) {
     if (groups < 1 || groups > 3 || rows <= 0 || K <= 0 || Ng <= 0) {
         set_error("proj_gemm: bad shape groups=%d rows=%ld K=%d N=%d", groups, rows, K, Ng);
         return 1;
@@ -804,8 +830,14 @@ int launch_proj_gemm(const void* x, const void* w, const float* bias, void* cons
         set_error("proj_gemm: tile_n must be 128 or 256");
         return 1;
     }
-    if (K % kPChunkK || Ng % tile_n || (long)K * 2 * kPTileR > 0x7fffffffL) {
-        set_error("proj_gemm: shape K=%d N=%d not supported (K %% 64, N %% %d)", K, Ng, tile_n);
+    if (in_dtype == 0 && (tile_n != 128 || out_dtype != 0)) {
+        set_error("proj_gemm: fp32 operands need tile_n 128 and fp32 output");
+        return 1;
+    }
+    const long kbytes = (long)K * (in_dtype == 0 ? 4 : 2);
+    if (kbytes % kPRowBytes || Ng % tile_n || kbytes * kPTileR > 0x7fffffffL) {
+        set_error("proj_gemm: shape K=%d N=%d not supported (K %% %d, N %% %d)", K, Ng,
+                  in_dtype == 0 ? kPChunkK / 2 : kPChunkK, tile_n);
         return 2;
     }
     if (accumulate && out_dtype != 0) {
@@ -836,8 +868,8 @@ int launch_proj_gemm(const void* x, const void* w, const float* bias, void* cons
         return 1;
     }
     ProjArgs a;
-    a.x = static_cast<const __bf16*>(x);
-    a.w = static_cast<const __bf16*>(w);
+    a.x = x;
+    a.w = w;
     a.bias = bias;
     for (int g = 0; g < 3; ++g) a.out[g] = g < groups ? outs[g] : nullptr;
     a.rows = rows;
@@ -847,7 +879,12 @@ int launch_proj_gemm(const void* x, const void* w, const float* bias, void* cons
     a.n_tiles = (int)n_tiles;
     a.r_tiles = (int)r_tiles;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (tile_n == 256) {
+    if (in_dtype == 0) {
+        if (accumulate)
+            launch_small<float, float, true>(a, st);
+        else
+            launch_small<float, float, false>(a, st);
+    } else if (tile_n == 256) {
         if (out_dtype == 1)
             launch_large<__bf16, false>(a, st);
         else if (accumulate)
@@ -856,11 +893,11 @@ int launch_proj_gemm(const void* x, const void* w, const float* bias, void* cons
             launch_large<float, false>(a, st);
     } else {
         if (out_dtype == 1)
-            launch_small<__bf16, false>(a, st);
+            launch_small<__bf16, __bf16, false>(a, st);
         else if (accumulate)
-            launch_small<float, true>(a, st);
+            launch_small<__bf16, float, true>(a, st);
         else
-            launch_small<float, false>(a, st);
+            launch_small<__bf16, float, false>(a, st);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -876,7 +913,7 @@ extern "C" int kvp_proj_gemm(const void* x, const void* w, const float* bias, vo
                              void* out1, void* out2, int groups, long rows, int K, int N,
                              int out_dtype, int accumulate, int tile_n, void* stream) {
     void* outs[3] = {out0, out1, out2};
-    const int rc = kvp::launch_proj_gemm(x, w, bias, outs, groups, rows, K, N, out_dtype,
+    const int rc = kvp::launch_proj_gemm(1, x, w, bias, outs, groups, rows, K, N, out_dtype,
                                          accumulate != 0, tile_n, stream);
     return rc == 0 ? 0 : 1;
 }

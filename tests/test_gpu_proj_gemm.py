@@ -90,3 +90,50 @@ def test_proj_gemm_rejects_unsupported_shapes(lib):
     assert lib.kvp_proj_gemm(16, 16, None, 16, None, None, 4, 4, 64, 256, 1, 0, 256, None) != 0
     assert lib.kvp_proj_gemm(16, 16, None, 16, None, None, 2, 4, 64, 256, 1, 0, 256, None) != 0
     assert lib.kvp_proj_gemm(16, 16, None, 16, None, None, 1, 4, 64, 256, 1, 0, 64, None) != 0
+
+
+# fp32 operands on the tiled kernel: one and many K chunks of 32, one row, the
+# edges of a 128-row tile, several feature tiles, both forms
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N,acc,bias", [
+    (1, 32, 128, False, True), (127, 64, 128, True, True), (128, 96, 256, False, False),
+    (129, 32, 128, True, False), (1560, 1536, 1536, False, True), (300, 1536, 384, True, True),
+])
+def test_fp32_linear_tiled(rows, K, N, acc, bias):
+    print(f"fp32 linear rows={rows} K={K} N={N} acc={acc}", flush=True)
+    rng = np.random.default_rng(rows + K + N)
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((N, K))).astype(np.float32)
+    b = (0.1 * rng.standard_normal(N)).astype(np.float32) if bias else None
+    y0 = rng.standard_normal((rows + 3, N)).astype(np.float32)
+    y = torch.from_numpy(y0).to(DEV)
+    kb.linear(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV),
+              None if b is None else torch.from_numpy(b).to(DEV), y[:rows], accumulate=acc)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.array_equal(got[rows:], y0[rows:]), "rows past the end were written"
+    want = ob.linear(x, w, b) + (y0[:rows] if acc else 0)
+    # each value is a chain of at most K + 2 rounded fp32 additions of terms
+    # whose magnitudes sum to |x| |w|^T + |b| + |y0|
+    mag = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    mag += (0 if b is None else np.abs(b)) + (np.abs(y0[:rows]) if acc else 0)
+    assert (np.abs(got[:rows] - want) <= (K + 2) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,heads", [(1, 1), (131, 3)])
+def test_fp32_qkv_project_is_three_linears(rows, heads):
+    """The grouped fp32 launch equals three single launches of its weight blocks, bit for bit."""
+    D = 128 * heads
+    print(f"fp32 qkv rows={rows} D={D}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, D, generator=g, device=DEV)
+    w = 0.02 * torch.randn(3 * D, D, generator=g, device=DEV)
+    b = torch.randn(3 * D, generator=g, device=DEV)
+    ln_w, ln_b = torch.ones(D, device=DEV), torch.zeros(D, device=DEV)
+    xn, q, k, v = (torch.empty(rows, D, device=DEV) for _ in range(4))
+    kb.qkv_project(x, ln_w, ln_b, w, b, xn, q, k, v)
+    for i, got in enumerate((q, k, v)):
+        want = torch.empty(rows, D, device=DEV)
+        kb.linear(xn, w[i * D:(i + 1) * D], b[i * D:(i + 1) * D], want)
+        assert torch.equal(got, want), i
