@@ -349,17 +349,15 @@ def producer_cpu_baseline(model, cfg, frames, layers):
                       f"1 layer, median of 3, x {layers} layers"}
 
 
-# Algorithmic HBM bytes per pixel of one full-size (level 0) launch, per frame
-# (pyramid kinds) or per pair (flow kinds); fp32 planes, uint8 frames.
+# Algorithmic HBM bytes per pixel of one full-size (level 0) pass, per frame
+# (expansion) or per pair (flow kinds); fp32 planes, uint8 frames. box_flow is
+# a whole iteration: flow and both frames' expansions in, flow out.
 MOTION_BYTES_PER_PX = {
-    "blur_rows": 1 + 4,               # uint8 frame in, fp32 row-blurred out
-    "blur_cols_resize": 4 + 4,        # fp32 in, fp32 level image out
-    "poly_exp": 4 + 5 * 4,            # image in, 5 expansion planes out
-    "matrices_init": 2 + 5 * 4 * 2 + 5 * 4,  # coarse flow (1/4 px), R0 + R1, M out
-    "box_flow": 5 * 4 + 2 * 4,        # M in, flow out
-    "matrices": 2 * 4 + 5 * 4 * 2 + 5 * 4,   # flow, R0 + R1, M out
+    "poly_exp": 1 + 5 * 4,            # uint8 frame in, 5 expansion values out
+    "matrices_init": 2 + 2 * 4,       # coarse flow (1/4 px), initial flow out
+    "box_flow": 2 * 4 + 5 * 4 * 2 + 2 * 4,
 }
-MOTION_PER_FRAME = ("blur_rows", "blur_cols_resize", "poly_exp")
+MOTION_PER_FRAME = ("poly_exp",)
 
 
 def motion_bench(args, torch, stream):
@@ -372,8 +370,8 @@ def motion_bench(args, torch, stream):
     Whole clip: W warmup, K timed runs (HIP events on the launch stream).
     Per launch: one run of kvp_farneback_profile (an event after every
     launch); the kind with the most time at level 0 is the dominant kernel,
-    its achieved bandwidth = algorithmic bytes of one level-0 launch / its
-    average level-0 duration."""
+    its achieved bandwidth = algorithmic bytes of one level-0 pass over the
+    clip / the average duration of its passes."""
     from kvpersist import motion, workloads
 
     n, H, W = args.motion_frames, 480, 832
@@ -407,16 +405,18 @@ def motion_bench(args, torch, stream):
     P, pairs = H * W, n - 1
 
     def level0_roof(kind):
+        # a level-0 pass over the clip may be several launches (chunks of pairs)
         units = n if kind in MOTION_PER_FRAME else pairs
+        passes = motion.FARNEBACK["iterations"] if kind == "box_flow" else 1
         nbytes = MOTION_BYTES_PER_PX[kind] * P * units
-        ms = sum(lvl0[kind]) / len(lvl0[kind])
+        ms = sum(lvl0[kind]) / passes
         ach = nbytes / (ms * 1e-3) / 1e9
         return {"bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach / HBM_PEAK_GBS, 4), "avg_launch_ms": round(ms, 5),
-                "launches_per_clip": len(lvl0[kind]),
-                "bytes_per_launch": nbytes,
-                "per_launch": f"{MOTION_BYTES_PER_PX[kind]} B/px x {P} px x {units} "
-                              f"{'frames' if kind in MOTION_PER_FRAME else 'pairs'}"}
+                "frac": round(ach / HBM_PEAK_GBS, 4), "avg_pass_ms": round(ms, 5),
+                "passes_per_clip": passes, "launches_per_clip": len(lvl0[kind]),
+                "bytes_per_pass": nbytes,
+                "per_pass": f"{MOTION_BYTES_PER_PX[kind]} B/px x {P} px x {units} "
+                            f"{'frames' if kind in MOTION_PER_FRAME else 'pairs'}"}
 
     # fabric bytes of the level-0 launches from rocprofv3 FETCH_SIZE / WRITE_SIZE
     # runs of this workload, scaled by a copy-kernel calibration (committed)
@@ -425,7 +425,7 @@ def motion_bench(args, torch, stream):
     if tfile.exists():
         try:
             rec = json.loads(tfile.read_text())["kernels"].get(dominant)
-            traffic = rec["hbm_bytes_per_launch"] if rec else None
+            traffic = rec["hbm_bytes_per_pass"] if rec else None
         except (OSError, ValueError, KeyError):
             traffic = None
     out = {

@@ -58,10 +58,12 @@ int kvp_farneback_flow(const unsigned char* prev, const unsigned char* next,
 
 /* kvp_farneback_flows with an event after every kernel launch, for
  * measurement (no counterpart in the reference, whose flow is a cv2 call):
- * launch i took launch_ms[i] on `stream`; launch_kind[i] is 0 pre-blur rows,
- * 1 pre-blur columns + resize, 2 polynomial expansion, 3 first matrix update
- * of a level (initial flow), 4 box filter + flow solve, 5 matrix update;
- * launch_level[i] is the pyramid level (0 = full size). Synchronises the
+ * launch i took launch_ms[i] on `stream`; launch_kind[i] is 1 pre-blur +
+ * resize, 2 polynomial expansion, 3 initial flow of a level, 4 flow (a whole
+ * iteration for window sizes 14 and 15; otherwise box filter + solve), 5 matrix
+ * update (other window sizes); 0 is not used. launch_level[i] is the pyramid
+ * level (0 = full size), the lowest one of a launch that covers several; a
+ * level's pairs may be taken in several launches. Synchronises the
  * stream. *count receives the number of launches (an error if > capacity). */
 int kvp_farneback_profile(const unsigned char* frames, int num_frames,
                           int width, int height, double pyr_scale, int levels,

@@ -329,3 +329,26 @@ def test_bad_arguments_raise():
     rc = lib.kvp_farneback_flows(f.data_ptr(), 2, 64, 64, 0.5, 3, 15, 3, 5, 1.2, 0,
                                  ws.data_ptr(), 16, out.data_ptr(), None)
     assert rc != 0 and "workspace" in _lib.last_error()
+
+
+@pytest.mark.parametrize("frames", [2, 20])
+def test_clip_taken_in_chunks_equals_its_pairs_bitwise(frames):
+    """20 frames of 832x480 hold more pairs than one chunk of the full-size
+    level takes; 2 frames are a single chunk whose levels expand together."""
+    clip = torch.from_numpy(workloads.synthetic_clip(frames, 480, 832, seed=3)).to(DEV)
+    flows = motion.farneback_flows(clip)
+    for p in sorted({0, (frames - 1) // 2, frames - 2}):
+        assert torch.equal(flows[p], motion.calc_optical_flow_farneback(clip[p], clip[p + 1])), p
+
+
+@pytest.mark.parametrize("H,W,params", [
+    (230, 200, dict(pyr_scale=0.85, levels=12)),   # more levels than one pyramid launch takes
+    (420, 401, dict(pyr_scale=0.3, levels=2)),     # 25-tap pre-blur, odd width
+    (700, 720, dict(pyr_scale=0.05, levels=1)),    # source under a block too wide to stage
+    (46, 85, dict(levels=0)),                      # one column past a strip, whole batches of rows
+    (33, 84, dict(levels=0, poly_n=8, poly_sigma=2.0)),
+])
+def test_pyramid_and_strip_edges_match_oracle(H, W, params):
+    clip = workloads.synthetic_clip(2, H, W, seed=H)
+    got = motion.calc_optical_flow_farneback(clip[0], clip[1], **params).cpu().numpy()
+    _flow_ok(got, fb.calc_optical_flow_farneback(clip[0], clip[1], **params), f"{H}x{W} {params}")
