@@ -310,12 +310,12 @@ def producer_bench(args, torch, stream):
             "layer_norm": roof("hbm", ln_bytes, ln_ms, HBM_PEAK_GBS, "GB/s",
                                f"{ln_bytes} B (fp32 row in, bf16 row out, {rows} rows)"),
             "qkv_proj": roof("mfma", qkv_flops, qkv_ms, BF16_PEAK_TFLOPS, "TFLOP/s",
-                             f"proj_gemm_bf16_kernel, 3 groups in one launch, {qkv_flops} flop"),
+                             f"proj_gemm_wide_kernel, 3 groups in one launch, {qkv_flops} flop"),
             "attention": roof("mfma", att_flops, att_ms, BF16_PEAK_TFLOPS, "TFLOP/s",
                               f"attn_fwd_bf16_kernel intra-frame, {frames} frames, "
                               f"{att_flops} flop"),
             "out_proj": roof("mfma", out_flops, out_ms, BF16_PEAK_TFLOPS, "TFLOP/s",
-                             f"proj_gemm_small_kernel, 1 group, fp32 residual added in the epilogue, {out_flops} flop"),
+                             f"proj_gemm_wide_kernel, 1 group, fp32 residual added in the epilogue, {out_flops} flop"),
         },
     }
     if not args.no_cpu_baseline:

@@ -114,8 +114,8 @@ int fill_words(void* dst, long n, unsigned value, void* stream);
 // outs[g][r, n] = sum_k x[r, k] w[g*Ng + n, k] + bias[g*Ng + n]
 // (+ outs[g][r, n] when accumulate; fp32 output only). x, w of in_dtype (0 =
 // fp32, 1 = bf16); bias fp32 or null; out_dtype 0 = fp32, 1 = bf16 (fp32
-// operands: fp32 only); tile_n 128 (128 x 128 tiles, two workgroups per CU)
-// or 256 (bf16 operands: 256 x 256 tiles, one workgroup per CU).
+// operands: fp32 only); tile_n 128 (the tiles measured fastest for the
+// shape) or 256 (bf16 operands: 256 x 256 tiles).
 // Returns 0 on success, 2 when the shape is outside the kernel's tiling
 // (K % 64, fp32 K % 32, or Ng % tile_n), 1 on any other error.
 int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bias,

@@ -5,33 +5,25 @@
 // for groups g < G, with x [rows, K] and w [G*Ng, K] bf16 or fp32 row-major
 // (both K-contiguous), bias fp32, out_g [rows, Ng] bf16 or fp32 (fp32 may
 // accumulate into itself: the residual add of out_proj; fp32 operands give
-// fp32 outputs). One launch covers
-// every group, so the three q/k/v projections of a DiT block
-// (reference: src/backbone.py:13,18-19) run as one grid written straight to
-// three token-major outputs, and out_proj (src/backbone.py:22,32-33) adds
-// into the fp32 residual stream in its epilogue.
+// fp32 outputs). One launch covers every group, so the three q/k/v projections
+// of a DiT block (reference: src/backbone.py:13,18-19) run as one grid written
+// straight to three token-major outputs, and out_proj (src/backbone.py:22,
+// 32-33) adds into the fp32 residual stream in its epilogue.
 //
-// Two tilings share the operand layout below: the large-tile kernel (256 x
-// 256, one workgroup per CU) and the small-tile kernel (128 x 128, two
-// workgroups per CU, described at its definition), which is the faster one
-// at the backbone's shapes and the one the q/k/v projection uses. fp32 operands
-// always take the small tiles.
+// Two tilings share the operand layout below: 128 features x 128 tokens (four
+// waves, two workgroups per CU), and, for bf16 operands, 256 features x 256 or
+// 320 tokens (eight waves, one workgroup per CU). choose_tile says which.
 //
-// Work decomposition (large tiles):
-//   workgroup = 4 waves, output tile TN features x 256 tokens; wave (wn, wr)
-//   owns (TN/2) x 128 of it as (TN/64) x 4 blocks of 32x32 accumulated by
-//   v_mfma_f32_32x32x16_bf16 with A = w rows (features), B = x rows
-//   (tokens): lane l holds token (l % 32) of a block and features
-//   8*(v/4) + 4*(l/32) + v%4 in accumulator register v.
-//   K advances in chunks of 64: both operand chunks ([TN][64] and [256][64]
-//   bf16, 128-byte rows) arrive by buffer loads straight into a two-stage LDS
-//   ring, 16-byte chunks XOR-swizzled by ((row >> 1) & 7) so that the
-//   fragment reads (ds_read_b128, 16 rows per read phase) hit distinct banks.
-//   Per k-step each wave reads its TN/64 + 4 fragments one step ahead of the
-//   MFMAs; the next chunk's copies are all issued after the first k-step's
-//   leading MFMAs, and the chunk barrier sits between the two halves of the
-//   last k-step's MFMAs, so the next chunk's first fragment reads overlap
-//   MFMAs.
+// Common structure:
+//   wave (wn, wr) of a workgroup owns 64 features x 32 * JR tokens as 2 x JR
+//   blocks of 32x32 accumulated by v_mfma_f32_32x32x16_bf16 with A = w rows
+//   (features), B = x rows (tokens): lane l holds token (l % 32) of a block
+//   and features 8*(v/4) + 4*(l/32) + v%4 in accumulator register v.
+//   K advances in chunks of 128 bytes per row: both operand chunks arrive by
+//   buffer loads straight into a two-stage LDS ring, 16-byte pieces
+//   XOR-swizzled by ((row >> 1) & 7) so that the fragment reads
+//   (ds_read_b128, 16 rows per read phase) hit distinct banks. Fragments are
+//   read one k-step ahead of their MFMAs.
 //   The accumulators start at the bias. Epilogue: each wave stages its
 //   outputs (converted to the output type) 32 tokens at a time in LDS as
 //   token rows, then writes them (and, when accumulating, reads the
@@ -44,7 +36,7 @@
 //
 // Token rows past `rows` read as zeros (buffer bounds) and are not stored.
 // Requirements (checked on the host): K % 64 == 0 (fp32 operands: K % 32),
-// Ng % TN == 0, 16-byte aligned operands.
+// Ng % 128 == 0, 16-byte aligned operands.
 
 #include <hip/hip_runtime.h>
 
@@ -60,12 +52,14 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
 constexpr int kPThreads = 256;
-constexpr int kPTileR = 256;   // tokens per workgroup tile (large-tile kernel)
 constexpr int kPSmall = 128;   // features and tokens per tile (small-tile kernel)
 constexpr int kPChunkK = 64;   // K per LDS stage
 constexpr int kPRowBytes = kPChunkK * 2;
 constexpr int kPBand = 4;      // token tiles per scheduling band
+constexpr int kWThreads = 512; // wide-tile kernel: 8 waves
+constexpr int kWTileN = 256;   // and its features per tile
 constexpr int kPNumXcd = 8;
+constexpr int kPCus = 256;
 constexpr int kPBufFlags = 0x00020000;
 
 struct ProjArgs {
@@ -111,251 +105,13 @@ __device__ __forceinline__ int pj_xcd_remap(int bid, int n) {
     return xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
 }
 
-template <int TN, typename OutT, bool kAcc>
-__global__ __launch_bounds__(kPThreads, 1) void proj_gemm_bf16_kernel(ProjArgs a) {
-    constexpr int JN = TN / 64;                 // 32-feature blocks per wave
-    constexpr int kWBytes = TN * kPRowBytes;    // weight chunk bytes
-    constexpr int kXBytes = kPTileR * kPRowBytes;
-    constexpr int kWCopies = kWBytes / 1024 / 4;  // 1 KiB copies per wave per chunk
-    constexpr int kXCopies = kXBytes / 1024 / 4;
-    // stages: weights [2][kWBytes] then tokens [2][kXBytes]; the epilogue
-    // reuses the space as per-wave output staging
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * (kWBytes + kXBytes)];
-    auto w_stage = [&](int s) { return (unsigned)(uintptr_t)lds + (unsigned)(s * kWBytes); };
-    auto x_stage = [&](int s) {
-        return (unsigned)(uintptr_t)lds + (unsigned)(2 * kWBytes + s * kXBytes);
-    };
-
-    // ---- tile coordinates ----
-    const int lid = pj_xcd_remap((int)blockIdx.x, (int)gridDim.x);
-    const int band_tiles = kPBand * a.n_tiles;
-    const int band = lid / band_tiles;
-    const int in_band = lid % band_tiles;
-    const int band_r0 = band * kPBand;
-    int band_h = a.r_tiles - band_r0;
-    if (band_h > kPBand) band_h = kPBand;
-    const int rt = band_r0 + in_band % band_h;
-    const int nt = in_band / band_h;
-    const int tiles_per_group = a.Ng / TN;
-    const int g = nt / tiles_per_group;
-    const int n0 = (nt % tiles_per_group) * TN;  // feature offset within the group
-    const long r0 = (long)rt * kPTileR;
-
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int lq = lane & 31;
-    const int hh = lane >> 5;
-    const int wn = wave & 1;
-    const int wr = wave >> 1;
-
-    // ---- copy setup: instruction i of a wave fills 1 KiB = 8 rows ----
-    const unsigned kbytes = (unsigned)a.K * 2u;
-    const __bf16* wg_base = static_cast<const __bf16*>(a.w) + ((long)g * a.Ng + n0) * a.K;
-    const __bf16* xg_base = static_cast<const __bf16*>(a.x) + r0 * a.K;
-    long xrows = a.rows - r0;
-    if (xrows > kPTileR) xrows = kPTileR;
-    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<__bf16*>(wg_base), (short)0, (int)(TN * kbytes), kPBufFlags);
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<__bf16*>(xg_base), (short)0, (int)(xrows * (long)kbytes), kPBufFlags);
-    // rows of copy i: row = 8*(nwave_copies*wave + i) + lane/8; physical
-    // chunk lane%8 holds logical chunk (lane%8) ^ ((row >> 1) & 7), and
-    // (row >> 1) & 7 = (4*(i & 1) + lane/16) & 7 for every copy.
-    const unsigned pch = (unsigned)(lane & 7);
-    const unsigned lrow = (unsigned)(lane >> 3);
-    const unsigned swz_even = (unsigned)((lane >> 4) & 7);
-    const unsigned swz_odd = (unsigned)((4 + (lane >> 4)) & 7);
-    const unsigned coff_even = 16u * (pch ^ swz_even);
-    const unsigned coff_odd = 16u * (pch ^ swz_odd);
-
-    auto issue_w = [&](int i, int stage, unsigned kofs) {
-        const unsigned row = 8u * (unsigned)(kWCopies * wave + i) + lrow;
-        const unsigned vo = row * kbytes + ((i & 1) ? coff_odd : coff_even);
-        PJ_LDS void* d = (PJ_LDS void*)(uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane(
-            (int)(w_stage(stage) + 1024u * (unsigned)(kWCopies * wave + i)));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, d, 16, vo, (int)kofs, 0, 0);
-    };
-    auto issue_x = [&](int i, int stage, unsigned kofs) {
-        const unsigned row = 8u * (unsigned)(kXCopies * wave + i) + lrow;
-        const unsigned vo = row * kbytes + ((i & 1) ? coff_odd : coff_even);
-        PJ_LDS void* d = (PJ_LDS void*)(uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane(
-            (int)(x_stage(stage) + 1024u * (unsigned)(kXCopies * wave + i)));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, d, 16, vo, (int)kofs, 0, 0);
-    };
-    // copy c of the chunk (0 .. kWCopies + kXCopies - 1), weights first
-    auto issue_copy = [&](int c, int stage, unsigned kofs) {
-        if (c < kWCopies)
-            issue_w(c, stage, kofs);
-        else
-            issue_x(c - kWCopies, stage, kofs);
-    };
-
-    // ---- fragment addresses: row (lane % 32) of each 32-row block ----
-    const unsigned fs = (unsigned)((lq >> 1) & 7);
-    const unsigned w_row = (unsigned)(wn * (TN / 2) + lq) * kPRowBytes;
-    const unsigned x_row = (unsigned)(wr * 128 + lq) * kPRowBytes;
-    auto frag_off = [&](int ks) { return ((unsigned)(2 * ks + hh) ^ fs) << 4; };
-
-    constexpr int NF = JN + 4;
-    u32x4 fr[2][NF];
-    auto read_frags = [&](u32x4 (&f)[NF], int stage, int ks) {
-        const unsigned wa = w_stage(stage) + w_row + frag_off(ks);
-        const unsigned xa = x_stage(stage) + x_row + frag_off(ks);
-        f[0] = pj_lds_b128<0>(wa);
-        if constexpr (JN > 1) f[1] = pj_lds_b128<32 * kPRowBytes>(wa);
-        if constexpr (JN > 2) f[2] = pj_lds_b128<64 * kPRowBytes>(wa);
-        if constexpr (JN > 3) f[3] = pj_lds_b128<96 * kPRowBytes>(wa);
-        f[JN + 0] = pj_lds_b128<0>(xa);
-        f[JN + 1] = pj_lds_b128<32 * kPRowBytes>(xa);
-        f[JN + 2] = pj_lds_b128<64 * kPRowBytes>(xa);
-        f[JN + 3] = pj_lds_b128<96 * kPRowBytes>(xa);
-    };
-
-    // Accumulators start at the bias: its loads overlap the prologue's copy
-    // wait instead of stalling the epilogue.
-    f32x16 acc[JN][4];
-    {
-        const float* bias = a.bias ? a.bias + (long)g * a.Ng + n0 + wn * (TN / 2) : nullptr;
-#pragma unroll
-        for (int i = 0; i < JN; ++i) {
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const float4 b4 = bias ? *reinterpret_cast<const float4*>(bias + 32 * i + 8 * q4 +
-                                                                          4 * hh)
-                                       : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    acc[i][j][4 * q4 + 0] = b4.x;
-                    acc[i][j][4 * q4 + 1] = b4.y;
-                    acc[i][j][4 * q4 + 2] = b4.z;
-                    acc[i][j][4 * q4 + 3] = b4.w;
-                }
-            }
-        }
-    }
-
-    auto mfma_half = [&](const u32x4 (&f)[NF], int half) {
-#pragma unroll
-        for (int i = 0; i < JN; ++i)
-#pragma unroll
-            for (int j = 2 * half; j < 2 * half + 2; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    __builtin_bit_cast(bf16x8, f[i]), __builtin_bit_cast(bf16x8, f[JN + j]),
-                    acc[i][j], 0, 0, 0);
-    };
-
-    const int nk = a.K / kPChunkK;
-    constexpr int kCopies = kWCopies + kXCopies;
-
-    // prologue: chunk 0 into stage 0, its first fragments
-#pragma unroll
-    for (int c = 0; c < kCopies; ++c) issue_copy(c, 0, 0u);
-    pj_wait_vm0();
-    pj_barrier();
-    read_frags(fr[0], 0, 0);
-
-    for (int t = 0; t < nk; ++t) {
-        const int st = t & 1;
-        const bool more = t + 1 < nk;
-        const unsigned knext = (unsigned)(t + 1) * kPRowBytes;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            u32x4 (&cur)[NF] = fr[ks & 1];
-            u32x4 (&nxt)[NF] = fr[(ks + 1) & 1];
-            pj_lgkm_wait(cur);
-            if (ks < 3) read_frags(nxt, st, ks + 1);
-            __builtin_amdgcn_s_setprio(1);
-            mfma_half(cur, 0);
-            __builtin_amdgcn_s_setprio(0);
-            if (ks == 3 && more) {
-                // chunk t+1 has landed for every wave once all pass here; all
-                // reads of chunk t are complete (waited above)
-                pj_wait_vm0();
-                pj_barrier();
-                read_frags(nxt, st ^ 1, 0);
-            }
-            if (ks == 0 && more) {
-                // all of the next chunk's copies at once, as early as the ring
-                // allows: their latency, not their issue, is what stalls
-#pragma unroll
-                for (int c = 0; c < kCopies; ++c) issue_copy(c, st ^ 1, knext);
-            }
-            __builtin_amdgcn_s_setprio(1);
-            mfma_half(cur, 1);
-            __builtin_amdgcn_s_setprio(0);
-        }
-    }
-
-    // ---- epilogue: stage as token rows in LDS, row-contiguous store ----
-    constexpr int kFeat = TN / 2;                   // features per wave
-    constexpr int kEs = (int)sizeof(OutT);
-    constexpr int kRowB = kFeat * kEs + 16;         // padded staging row (bytes)
-    constexpr int kChunks = kFeat * kEs / 16;       // 16-byte chunks per row
-    constexpr int kRowsPerPass = 64 / kChunks;      // rows one wave instruction covers
-    static_assert(4 * 32 * kRowB <= 2 * (kWBytes + kXBytes), "staging exceeds LDS");
-    pj_barrier();  // every wave has finished reading the operand stages
-    OutT* out = static_cast<OutT*>(a.out[g]);
-    unsigned char* sbase = lds + wave * 32 * kRowB;
-    const int rchunk = lane % kChunks;
-    const int rrow = lane / kChunks;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        unsigned char* wrow = sbase + lq * kRowB;
-#pragma unroll
-        for (int i = 0; i < JN; ++i) {
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const float v0 = acc[i][j][4 * q4 + 0];
-                const float v1 = acc[i][j][4 * q4 + 1];
-                const float v2 = acc[i][j][4 * q4 + 2];
-                const float v3 = acc[i][j][4 * q4 + 3];
-                OutT* p = reinterpret_cast<OutT*>(wrow) + 32 * i + 8 * q4 + 4 * hh;
-                if constexpr (kEs == 4) {
-                    *reinterpret_cast<float4*>(p) = make_float4(v0, v1, v2, v3);
-                } else {
-                    struct alignas(8) B4 {
-                        __bf16 v[4];
-                    } o;
-                    o.v[0] = (__bf16)v0;
-                    o.v[1] = (__bf16)v1;
-                    o.v[2] = (__bf16)v2;
-                    o.v[3] = (__bf16)v3;
-                    *reinterpret_cast<B4*>(p) = o;
-                }
-            }
-        }
-        // same-wave LDS accesses complete in order: the rows written above
-        // are read back below, and the next block's writes follow these reads
-#pragma unroll
-        for (int pass = 0; pass < 32 / kRowsPerPass; ++pass) {
-            const int row = pass * kRowsPerPass + rrow;
-            const long r = r0 + wr * 128 + 32 * j + row;
-            const u32x4 vals = *reinterpret_cast<const u32x4*>(sbase + row * kRowB + 16 * rchunk);
-            if (r >= a.rows) continue;
-            unsigned char* gp = reinterpret_cast<unsigned char*>(out + r * a.Ng + n0 + wn * kFeat) +
-                                16 * rchunk;
-            if constexpr (kAcc) {
-                float4 y = *reinterpret_cast<const float4*>(gp);
-                y.x += __uint_as_float(vals[0]);
-                y.y += __uint_as_float(vals[1]);
-                y.z += __uint_as_float(vals[2]);
-                y.w += __uint_as_float(vals[3]);
-                *reinterpret_cast<float4*>(gp) = y;
-            } else {
-                *reinterpret_cast<u32x4*>(gp) = vals;
-            }
-        }
-    }
-}
-
 // Small-tile form: TN features x TR tokens per workgroup (128 x 128), two
-// workgroups per CU (64 KiB of LDS each: K chunks of 64 in a two-stage ring,
-// the same 128-byte swizzled rows as above); wave (wn, wr) owns (TN/2) x
-// (TR/2) as (TN/64) x (TR/64) blocks. Each chunk's copies are issued right
-// after the barrier that frees their stage. With two resident workgroups the
-// one in its epilogue or waiting on copies leaves the MFMA pipe to the other,
-// and four times as many tiles even out the rounds over the CUs.
+// workgroups per CU (64 KiB of LDS each); wave (wn, wr) owns (TN/2) x (TR/2) as
+// (TN/64) x (TR/64) blocks. Each chunk's copies are issued right after the
+// barrier that frees their stage. With two resident workgroups the one in its
+// epilogue or waiting on copies leaves the MFMA pipe to the other, and the many
+// tiles even out the rounds over the CUs. Bound by its copies: at full MFMA
+// rate its two workgroups would draw 64 bytes per cycle and CU from the L2.
 //
 // InT is the operands' type. A stage row is 128 bytes of K either way (64 bf16
 // or 32 fp32 values), so copies, swizzle and fragment reads are the same
@@ -543,7 +299,7 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_small_kernel(ProjArgs 
         }
     }
 
-    // epilogue: as in the large-tile kernel, 32 tokens at a time
+    // epilogue: 32 tokens at a time
     constexpr int kRowB = kFeat * kEs + 16;
     static_assert(4 * 32 * kRowB <= 2 * kSB, "staging exceeds LDS");
     if constexpr (kAcc) {
@@ -599,11 +355,288 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_small_kernel(ProjArgs 
     }
 }
 
-template <typename OutT, bool kAcc>
-void launch_large(const ProjArgs& a, hipStream_t st) {
-    const int grid = a.n_tiles * a.r_tiles;
-    hipLaunchKernelGGL((proj_gemm_bf16_kernel<256, OutT, kAcc>), dim3((unsigned)grid),
-                       dim3(kPThreads), 0, st, a);
+// Wide-tile form (bf16): 256 features x TR = 64 * JR tokens per workgroup of 8
+// waves, one workgroup per CU, two waves per SIMD. Wave (wn, wr) = (wave % 4,
+// wave / 4) owns 64 features x TR / 2 tokens as 2 x JR blocks. A tile of
+// 256 x 320 draws less than half the L2 bytes per MFMA of a 128 x 128 one. The
+// chunk barrier sits between the last k-step's MFMAs, so that the next chunk's
+// first fragments arrive under the rest of them, and the copies of a chunk
+// (2.5 us of MFMAs ahead of their use) are spread over the k-steps.
+// A tile may hold features of two groups (each wave's 64 lie in one) and reach
+// past the last group.
+//
+// 12,480 tokens, K = 1536: q/k/v 3 x 1536 features in 153 us (1,151 TFLOP/s;
+// 128 x 128 tiles: 205 us on the same GPU), out_proj + residual in 69 us (85).
+// Beyond the MFMAs a tile's epilogue and first chunk are exposed, with one
+// workgroup per CU.
+template <int JR, typename OutT, bool kAcc>
+__global__ __launch_bounds__(kWThreads, 2) void proj_gemm_wide_kernel(ProjArgs a) {
+    constexpr int TN = kWTileN, TR = 64 * JR, JN = 2;
+    constexpr int kWB = TN * kPRowBytes, kXB = TR * kPRowBytes, kSB = kWB + kXB;
+    constexpr int kWC = kWB / 8192, kXC = kXB / 8192, kCP = kWC + kXC;  // copies per wave
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kSB];
+
+    const int lid = pj_xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int band_tiles = kPBand * a.n_tiles;
+    const int band = lid / band_tiles;
+    const int in_band = lid % band_tiles;
+    const int band_r0 = band * kPBand;
+    int band_h = a.r_tiles - band_r0;
+    if (band_h > kPBand) band_h = kPBand;
+    const int rt = band_r0 + in_band % band_h;
+    const int n0 = in_band / band_h * TN;  // first feature, over all groups
+    const long r0 = (long)rt * TR;
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int lq = lane & 31;
+    const int hh = lane >> 5;
+    const int wn = wave & 3;
+    const int wr = wave >> 2;
+
+    const unsigned kbytes = (unsigned)a.K * 2u;
+    const int nall = a.groups * a.Ng;
+    const int wrows = min(nall - n0, TN);
+    long xrows = a.rows - r0;
+    if (xrows > TR) xrows = TR;
+    // rows past the features or tokens read as zeros
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<__bf16*>(static_cast<const __bf16*>(a.w) + (long)n0 * a.K), (short)0,
+        (int)((unsigned)wrows * kbytes), kPBufFlags);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<__bf16*>(static_cast<const __bf16*>(a.x) + r0 * a.K), (short)0,
+        (int)(xrows * (long)kbytes), kPBufFlags);
+    const unsigned lds0 = (unsigned)(uintptr_t)lds;
+    // copy c of a chunk: 1 KiB block blk of the weight (c < kWC) or token
+    // operand, rows 8*blk + lane/8, physical chunk lane % 8. Blocks of a wave
+    // are 8 apart, so that (row >> 1) & 7 is the same for all of them.
+    const unsigned crow = 8u * (unsigned)wave + (unsigned)(lane >> 3);
+    const unsigned cofs = crow * kbytes + 16u * ((unsigned)(lane & 7) ^ ((crow >> 1) & 7u));
+    auto issue_copy = [&](int c, int stage, unsigned kofs) {
+        const bool isw = c < kWC;
+        const unsigned blk = 8u * (unsigned)(isw ? c : c - kWC);
+        const unsigned dst = lds0 + (unsigned)(stage * kSB) + (isw ? 0u : (unsigned)kWB) +
+                             1024u * (blk + (unsigned)wave);
+        PJ_LDS void* d = (PJ_LDS void*)(uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)dst);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? wrs : xrs, d, 16, cofs + blk * 8u * kbytes,
+                                                 (int)kofs, 0, 0);
+    };
+    const unsigned fs = (unsigned)((lq >> 1) & 7);
+    const unsigned w_row = (unsigned)(wn * 64 + lq) * kPRowBytes;
+    const unsigned x_row = (unsigned)(wr * (TR / 2) + lq) * kPRowBytes;
+    constexpr int NF = JN + JR;
+    auto read_frags = [&](u32x4 (&f)[NF], int stage, int ks) {
+        const unsigned fo = ((unsigned)(2 * ks + hh) ^ fs) << 4;
+        const unsigned wa = lds0 + (unsigned)(stage * kSB) + w_row + fo;
+        const unsigned xa = lds0 + (unsigned)(stage * kSB + kWB) + x_row + fo;
+        f[0] = pj_lds_b128<0>(wa);
+        f[1] = pj_lds_b128<32 * kPRowBytes>(wa);
+        f[JN] = pj_lds_b128<0>(xa);
+        f[JN + 1] = pj_lds_b128<32 * kPRowBytes>(xa);
+        f[JN + 2] = pj_lds_b128<64 * kPRowBytes>(xa);
+        f[JN + 3] = pj_lds_b128<96 * kPRowBytes>(xa);
+        if constexpr (JR > 4) f[JN + 4] = pj_lds_b128<128 * kPRowBytes>(xa);
+    };
+    static_assert(JR == 4 || JR == 5, "fragment reads cover 4 or 5 token blocks");
+
+    // a wave's 64 features lie in one group (Ng is a multiple of 128)
+    const int nw = n0 + wn * 64;
+    const int g = min(nw / a.Ng, a.groups - 1);
+    const int ng = nw - g * a.Ng;  // feature within the group
+    f32x16 acc[JN][JR];
+    {
+        const float* bias = a.bias && nw < nall ? a.bias + nw : nullptr;
+#pragma unroll
+        for (int i = 0; i < JN; ++i) {
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const float4 b4 = bias ? *reinterpret_cast<const float4*>(bias + 32 * i + 8 * q4 +
+                                                                          4 * hh)
+                                       : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (int j = 0; j < JR; ++j) {
+                    acc[i][j][4 * q4 + 0] = b4.x;
+                    acc[i][j][4 * q4 + 1] = b4.y;
+                    acc[i][j][4 * q4 + 2] = b4.z;
+                    acc[i][j][4 * q4 + 3] = b4.w;
+                }
+            }
+        }
+    }
+    const int nk = (int)(kbytes / kPRowBytes);
+#pragma unroll
+    for (int c = 0; c < kCP; ++c) issue_copy(c, 0, 0u);
+    pj_wait_vm0();
+    pj_barrier();
+    u32x4 fr[2][NF];
+    read_frags(fr[0], 0, 0);
+    auto mfma = [&](const u32x4 (&f)[NF], int j0, int j1) {
+#pragma unroll
+        for (int j = j0; j < j1; ++j)
+#pragma unroll
+            for (int i = 0; i < JN; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, f[i]), __builtin_bit_cast(bf16x8, f[JN + j]),
+                    acc[i][j], 0, 0, 0);
+    };
+    for (int t = 0; t < nk; ++t) {
+        const int st = t & 1;
+        const bool more = t + 1 < nk;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            u32x4 (&cur)[NF] = fr[ks & 1];
+            u32x4 (&nxt)[NF] = fr[(ks + 1) & 1];
+            pj_lgkm_wait(cur);
+            if (ks < 3) read_frags(nxt, st, ks + 1);
+            // the next chunk's copies, spread over the first k-steps: their
+            // stage was last read before the barrier of the previous chunk
+            if (ks < 3 && more) {
+#pragma unroll
+                for (int c = ks * kCP / 3; c < (ks + 1) * kCP / 3; ++c)
+                    issue_copy(c, st ^ 1, (unsigned)(t + 1) * kPRowBytes);
+            }
+            __builtin_amdgcn_s_setprio(1);
+            if (ks < 3) {
+                mfma(cur, 0, JR);
+            } else {
+                // the chunk barrier sits between the last k-step's MFMAs: every
+                // read of chunk t is complete (waited above), and once all
+                // waves pass here chunk t+1 has landed; its first fragments
+                // arrive under the remaining MFMAs
+                mfma(cur, 0, JR / 2);
+                if (more) {
+                    pj_wait_vm0();
+                    pj_barrier();
+                    read_frags(nxt, st ^ 1, 0);
+                }
+                mfma(cur, JR / 2, JR);
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+    }
+
+    // epilogue: 32 tokens x 64 features of a wave at a time, staged in LDS as
+    // token rows and stored as full 16-byte lanes along rows
+    constexpr int kFeat = 64;
+    constexpr int kEs = (int)sizeof(OutT);
+    constexpr int kChunks = kFeat * kEs / 16;
+    constexpr int kRowsPerPass = 64 / kChunks;
+    constexpr int kPasses = 32 / kRowsPerPass;
+    constexpr int kRowB = kFeat * kEs + 16;
+    static_assert(8 * 32 * kRowB <= 2 * kSB, "staging exceeds LDS");
+    OutT* out = static_cast<OutT*>(a.out[g]);
+    const int rchunk = lane % kChunks;
+    const int rrow = lane / kChunks;
+    float4 resid[kAcc ? 2 : 1][kAcc ? kPasses : 1];
+    auto load_resid = [&](int j) {
+#pragma unroll
+        for (int pass = 0; pass < kPasses; ++pass) {
+            const long r = r0 + wr * (TR / 2) + 32 * j + pass * kRowsPerPass + rrow;
+            const long rc = r < a.rows ? r : a.rows - 1;
+            if (nw < nall)
+                resid[j & 1][pass] = *reinterpret_cast<const float4*>(
+                    reinterpret_cast<const float*>(out) + rc * a.Ng + ng + 4 * rchunk);
+        }
+    };
+    if constexpr (kAcc) load_resid(0);
+    pj_barrier();  // every wave has finished reading the operand stages
+    if (nw >= nall) return;
+    unsigned char* sbase = lds + wave * 32 * kRowB;
+#pragma unroll
+    for (int j = 0; j < JR; ++j) {
+        if constexpr (kAcc) {
+            if (j + 1 < JR) load_resid(j + 1);
+        }
+        unsigned char* wrow = sbase + lq * kRowB;
+#pragma unroll
+        for (int i = 0; i < JN; ++i) {
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const float v0 = acc[i][j][4 * q4 + 0];
+                const float v1 = acc[i][j][4 * q4 + 1];
+                const float v2 = acc[i][j][4 * q4 + 2];
+                const float v3 = acc[i][j][4 * q4 + 3];
+                OutT* p = reinterpret_cast<OutT*>(wrow) + 32 * i + 8 * q4 + 4 * hh;
+                if constexpr (kEs == 4) {
+                    *reinterpret_cast<float4*>(p) = make_float4(v0, v1, v2, v3);
+                } else {
+                    struct alignas(8) B4 {
+                        __bf16 v[4];
+                    } o;
+                    o.v[0] = (__bf16)v0;
+                    o.v[1] = (__bf16)v1;
+                    o.v[2] = (__bf16)v2;
+                    o.v[3] = (__bf16)v3;
+                    *reinterpret_cast<B4*>(p) = o;
+                }
+            }
+        }
+#pragma unroll
+        for (int pass = 0; pass < kPasses; ++pass) {
+            const int row = pass * kRowsPerPass + rrow;
+            const long r = r0 + wr * (TR / 2) + 32 * j + row;
+            const u32x4 vals = *reinterpret_cast<const u32x4*>(sbase + row * kRowB + 16 * rchunk);
+            if (r >= a.rows) continue;
+            unsigned char* gp =
+                reinterpret_cast<unsigned char*>(out + r * a.Ng + ng) + 16 * rchunk;
+            if constexpr (kAcc) {
+                float4 y = resid[j & 1][pass];
+                y.x += __uint_as_float(vals[0]);
+                y.y += __uint_as_float(vals[1]);
+                y.z += __uint_as_float(vals[2]);
+                y.w += __uint_as_float(vals[3]);
+                *reinterpret_cast<float4*>(gp) = y;
+            } else {
+                *reinterpret_cast<u32x4*>(gp) = vals;
+            }
+        }
+    }
+}
+
+template <int JR, typename OutT, bool kAcc>
+void launch_wide(ProjArgs a, hipStream_t st) {
+    a.n_tiles = (a.groups * a.Ng + kWTileN - 1) / kWTileN;
+    a.r_tiles = (int)((a.rows + 64 * JR - 1) / (64 * JR));
+    hipLaunchKernelGGL((proj_gemm_wide_kernel<JR, OutT, kAcc>),
+                       dim3((unsigned)(a.n_tiles * a.r_tiles)), dim3(kWThreads), 0, st, a);
+}
+
+template <int JR>
+void launch_wide(const ProjArgs& a, int out_dtype, bool accumulate, hipStream_t st) {
+    if (out_dtype == 1)
+        launch_wide<JR, __bf16, false>(a, st);
+    else if (accumulate)
+        launch_wide<JR, float, true>(a, st);
+    else
+        launch_wide<JR, float, false>(a, st);
+}
+
+// Tile of a bf16 launch: 0 = 128 x 128, else JR of the wide form (4: 256 x 256,
+// 5: 256 x 320). Each form's time is its rounds over the chip times the measured
+// time of a round (K = 1536; every term scales with K alike): 128 x 128 fills
+// 512 slots in 29 us, and its tiles even out beyond the first round; 256 x 256
+// takes 43.6 us a round of 256, 256 x 320 51 us. All three add the same terms
+// in the same order: results are equal bit for bit. Measured (us; 128 x 128,
+// 256 x 256, 256 x 320): 12480 tokens x 3 x 1536 features 205, 175, 153; x 1536
+// accumulating 85, 95, 69; 8000 x 3 x 1664 135, 132, 114; x 1664 65, 55, 62;
+// 5365 x 3 x 1152 52, 59, 42; 1560 x 3 x 1536 27, 38, 41.
+int choose_tile(long rows, int features) {
+    const double small_tiles =
+        (double)((rows + kPSmall - 1) / kPSmall) * ((features + kPSmall - 1) / kPSmall);
+    double best = 29.0 * (small_tiles > 2 * kPCus ? small_tiles / (2 * kPCus) : 1.0);
+    int jr = 0;
+    const double round_us[2] = {43.6, 51.0};
+    for (int j = 4; j <= 5; ++j) {
+        const long tiles =
+            ((rows + 64 * j - 1) / (64 * j)) * ((features + kWTileN - 1) / kWTileN);
+        const double t = round_us[j - 4] * (double)((tiles + kPCus - 1) / kPCus);
+        if (t < best) {
+            best = t;
+            jr = j;
+        }
+    }
+    return jr;
 }
 
 template <typename InT, typename OutT, bool kAcc>
@@ -835,7 +868,7 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
         return 1;
     }
     const long kbytes = (long)K * (in_dtype == 0 ? 4 : 2);
-    if (kbytes % kPRowBytes || Ng % tile_n || kbytes * kPTileR > 0x7fffffffL) {
+    if (kbytes % kPRowBytes || Ng % tile_n || kbytes * kWTileN > 0x7fffffffL) {
         set_error("proj_gemm: shape K=%d N=%d not supported (K %% %d, N %% %d)", K, Ng,
                   in_dtype == 0 ? kPChunkK / 2 : kPChunkK, tile_n);
         return 2;
@@ -860,10 +893,9 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
         set_error("proj_gemm: operands must be 16-byte aligned");
         return 1;
     }
-    const long tile_r = tile_n == 256 ? kPTileR : kPSmall;
-    const long r_tiles = (rows + tile_r - 1) / tile_r;
-    const long n_tiles = (long)groups * (Ng / tile_n);
-    if (r_tiles * n_tiles > 0x7fffffffL) {
+    const long r_tiles = (rows + kPSmall - 1) / kPSmall;
+    const long n_tiles = (long)groups * (Ng / kPSmall);
+    if (r_tiles * n_tiles > 0x7fffffffL || (long)groups * Ng > 0x7fffffffL) {
         set_error("proj_gemm: grid too large");
         return 1;
     }
@@ -884,15 +916,15 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
             launch_small<float, float, true>(a, st);
         else
             launch_small<float, float, false>(a, st);
-    } else if (tile_n == 256) {
-        if (out_dtype == 1)
-            launch_large<__bf16, false>(a, st);
-        else if (accumulate)
-            launch_large<float, true>(a, st);
-        else
-            launch_large<float, false>(a, st);
     } else {
-        if (out_dtype == 1)
+        int jr = tile_n == 256 ? 4 : choose_tile(rows, groups * Ng);
+        // (a tile's tokens are addressed with 32-bit offsets)
+        if (64 * jr * kbytes > 0x7fffffffL) jr = 0;
+        if (jr == 5)
+            launch_wide<5>(a, out_dtype, accumulate, st);
+        else if (jr == 4)
+            launch_wide<4>(a, out_dtype, accumulate, st);
+        else if (out_dtype == 1)
             launch_small<__bf16, __bf16, false>(a, st);
         else if (accumulate)
             launch_small<__bf16, float, true>(a, st);

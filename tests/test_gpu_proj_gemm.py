@@ -137,3 +137,17 @@ def test_fp32_qkv_project_is_three_linears(rows, heads):
         want = torch.empty(rows, D, device=DEV)
         kb.linear(xn, w[i * D:(i + 1) * D], b[i * D:(i + 1) * D], want)
         assert torch.equal(got, want), i
+
+
+# the wide tiles: tokens that end inside a tile of 320 or 256, feature tiles that
+# hold two groups and reach past the last one, one and several K chunks
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N,groups,tile_n,out_dt,acc,bias", [
+    (12473, 64, 1408, 3, 128, 1, False, True),
+    (12473, 192, 1536, 1, 128, 0, True, True),
+    (12473, 128, 384, 3, 128, 0, False, False),
+    (255, 128, 256, 3, 256, 1, False, True),
+    (513, 64, 512, 1, 256, 0, True, True),
+])
+def test_wide_tiles_match_oracle(rows, K, N, groups, tile_n, out_dt, acc, bias):
+    test_proj_gemm_matches_oracle(rows, K, N, groups, tile_n, out_dt, acc, bias)
