@@ -42,6 +42,8 @@
 #include <cstdio>
 #include <mutex>
 #include <thread>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "kvp_c_api.h"
@@ -58,6 +60,17 @@ typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 
 constexpr int kHeadDim = 128;
 constexpr int kThreads = 256;
+
+// f(0) .. f(N - 1) with compile-time indices
+template <int... I, typename F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
 constexpr int kBlockQ = 128;  // 4 waves x 32 queries
 constexpr int kNumXcd = 8;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -265,8 +278,9 @@ __device__ __forceinline__ float softmax_update(float (&s)[N], float scale_log2,
 // bf16 kernel
 //
 // K and V tiles (64 keys x 128 dims, 16 KiB each) stream global -> LDS with
-// buffer_load_dwordx4 ... lds (no register staging) into a two-stage ring:
-// the loads of tile t+1 are in flight while tile t is computed. Lane l of the
+// buffer_load_dwordx4 ... lds (no register staging) into rings of two (K) and
+// three (V) stages: the loads of tile t+1 are in flight while tile t is
+// computed. 80 KiB of LDS: two workgroups per CU. Lane l of the
 // wave's load instruction writes LDS bytes [base + 16*l, +16); it picks the
 // global 16-byte chunk that belongs at that (swizzled) LDS position.
 //
@@ -301,10 +315,6 @@ constexpr int kBufFlags = 0x00020000;
 // softmax note above).
 constexpr float kRowSumLimit = (float)kBf16BlockKeys;
 constexpr unsigned kVSwzTable = 0xAC60u;  // nibbles {0, 6, 12, 10}
-// Buffer offset past the records of every bf16 tile descriptor (a tile
-// covers at most 64 rows of 2*D bytes): a load there reads no memory and
-// returns zeros.
-constexpr unsigned kNoRecord = 0x80000000u;
 
 typedef __attribute__((ext_vector_type(4))) short v4i16;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
@@ -365,10 +375,6 @@ __device__ __forceinline__ u32x2 lds_tr16(unsigned addr) {
     return r;
 }
 
-__device__ __forceinline__ void lgkm_wait2(u32x4& a, u32x4& b) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b)::"memory");
-}
-
 // Waits for all but the two most recent LDS reads (LDS reads complete in
 // issue order and no scalar-memory load is issued in the compute phase).
 __device__ __forceinline__ void lgkm_wait2_keep2(u32x4& a, u32x4& b) {
@@ -392,8 +398,8 @@ __device__ __forceinline__ void lgkm_wait16(unsigned (&d)[16]) {
 
 // Waits until at most N LDS reads are outstanding.
 template <int N>
-__device__ __forceinline__ void lgkm_wait_tr_n(u32x2& a, u32x2& b, u32x2& c, u32x2& d) {
-    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "n"(N) : "memory");
+__device__ __forceinline__ void lgkm_wait_n(u32x2& a, u32x2& b) {
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N) : "memory");
 }
 
 // bf16 kernel epilogue: the wave's 32 query rows x 128 dims go out as
@@ -482,14 +488,13 @@ template <typename OutT, bool kMap, bool kColdNt, bool kCyclic, bool kGd = false
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) {
     static_assert(!kGd || (kMap && !kColdNt), "group descriptors serve the KVMap kernel");
     constexpr int kColdAux = kColdNt ? 2 : 0;  // buffer-load aux: bit 1 = nt
-    __shared__ __attribute__((aligned(1024))) unsigned char k_lds0[kBf16TileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char v_lds0[kBf16TileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char k_lds1[kBf16TileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char v_lds1[kBf16TileBytes];
-    // Per-wave 2 KiB sink (KVMap kernel): the interleaved copies of a group
-    // mixing arena and original rows land there (reading nothing), while
-    // the group's own rows come from its per-lane copies.
-    __shared__ __attribute__((aligned(1024))) unsigned char sink_lds[kMap ? 4 * 2048 : 16];
+    // K in a ring of two stages, V in three: a tile's PV product runs under the
+    // next tile's softmax, so its V stays for one more step.
+    constexpr int kVStages = 3;
+    __shared__
+        __attribute__((aligned(1024))) unsigned char lds[(2 + kVStages) * kBf16TileBytes];
+    unsigned char* const k_lds = lds;
+    unsigned char* const v_lds = lds + 2 * kBf16TileBytes;
 
     const WgCoord c = decode_wg(a);
     if (!c.valid) return;  // whole workgroup: past the end of the layer order
@@ -725,17 +730,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     // pair after every second QK k-step of the tile being computed, so the
     // copies trickle out between MFMAs (copy_plain).
     // copy_plain(i) reads K at cp_k + i*cp_step + kofs[i] and V at
-    // cp_v + i*cp_step + vofs through krs / vrs into LDS bytes pk + i*pstep
-    // and pv + i*pstep. For a plain group (no KVMap entry) krs / vrs cover
-    // the tile's K / V rows; for a run they both start at the run's first
-    // arena row; for a mixed group (copy_pair fills its rows) the offsets lie
-    // past the tile's records, so these copies read nothing, and they land
-    // in the wave's sink.
+    // cp_v + i*cp_step + vofs through krs / vrs into LDS bytes koff + 1024*i
+    // and voff + 1024*i. For a run krs / vrs both start at the run's first
+    // arena row; for every other group they cover the tile's K / V rows, and
+    // copy_pair replaces the rows that a mixed group has in the arena.
     __amdgpu_buffer_rsrc_t krs, vrs;
     unsigned koff = 0, voff = 0;
     unsigned cp_k = lane_row, cp_v = lane_row, cp_step = 4u * rb;
-    unsigned pk = 0, pv = 0, pstep = 1024u;
-    const unsigned sink = (unsigned)(uintptr_t)sink_lds + 2048u * (unsigned)wave;
     const unsigned lane_arena_v = lane_arena + rb;
     // step i's tile starts kvo bytes into the frame's K / V
     auto prep_tile = [&](int i, long kvo, unsigned char* kdst, unsigned char* vdst) {
@@ -753,9 +754,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
         cp_k = lane_row;
         cp_v = lane_row;
         cp_step = 4u * rb;
-        pk = koff;
-        pv = voff;
-        pstep = 1024u;
         if (kRuns && grp_run) {
             // a run's [K row | V row] arena rows: 2*rb apart, V rb after K
             krs = __builtin_amdgcn_make_buffer_rsrc(
@@ -764,18 +762,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             cp_k = lane_arena;
             cp_v = lane_arena_v;
             cp_step = 8u * rb;
-        } else if (kMap && grp_mapped) {
-            cp_k = kNoRecord;
-            cp_v = kNoRecord;
-            cp_step = 0;
-            pk = sink;
-            pv = sink + 1024u;
-            pstep = 0;
         }
     };
     auto copy_plain = [&](int i) {
-        KVP_LDS void* kd = (KVP_LDS void*)(uintptr_t)(pk + pstep * (unsigned)i);
-        KVP_LDS void* vd = (KVP_LDS void*)(uintptr_t)(pv + pstep * (unsigned)i);
+        KVP_LDS void* kd = (KVP_LDS void*)(uintptr_t)(koff + 1024u * (unsigned)i);
+        KVP_LDS void* vd = (KVP_LDS void*)(uintptr_t)(voff + 1024u * (unsigned)i);
         const unsigned step = (unsigned)i * cp_step;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, kd, 16, cp_k + step + kofs[i], 0, 0,
                                                  kColdAux);
@@ -832,24 +823,78 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     const int vsub = 8 * (tr_r & 1);
     const unsigned vcl = (unsigned)(2 * (grp & 1) + (tr_r >> 1));  // chunk bits below 4*nb
 
-    // `between(ks)` runs after the MFMAs of QK k-step ks (the next tile's
-    // copies are issued there).
-    auto compute_tile = [&](int t, const unsigned char* ks_lds, const unsigned char* vt_lds,
-                            auto&& between) {
+    // One step of the loop: the scores of its tile, then its softmax with the
+    // PV product of the tile before (V at v_prev, P in pd) between the
+    // exponentials, MFMA by MFMA. `between(ks)` runs after the MFMAs of QK
+    // k-step ks (the next tile's copies are issued there), `after` once the
+    // scores' MFMAs are issued.
+    // Bound by the wave's instruction issue and the CU's power, not by memory:
+    // QK, softmax and PV of one tile depend on each other, so a wave that takes
+    // them in turn leaves the matrix core to the CU's other workgroup for a
+    // third of its time. Its only independent work is the tile before:
+    // MFMA + FMA + exponential + pack interleaved take 35 cycles, the MFMA
+    // alone 32.5, so the scheduling barriers keep the order written here.
+    // Before -> after (PV under its own tile's step -> under the next): 21
+    // causal frames x 3600 tokens, 12 heads, 16.79 -> 15.07 ms (1.22 PFLOP/s,
+    // the rate of a large library bf16 product on the same card); 8 frames
+    // within themselves, 1560 tokens, 131 -> 126 us; 8 causal steps through
+    // the map 689 -> 648 us. Waves of 64 queries, one per SIMD, on the same
+    // schedule: 16.3 ms and 153 us.
+    // The values and the order in which they are added to O are those of the
+    // product taken in the tile's own step. The first step's pending product
+    // is 0 x 0.
+    u32x4 pd[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) pd[g] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < kBf16TileBytes / 16 / kThreads; ++i)
+        *reinterpret_cast<u32x4*>(v_lds + 2 * kBf16TileBytes + 16 * (tid + kThreads * i)) =
+            u32x4{0u, 0u, 0u, 0u};
+    // V^T fragment j = 4 g + nb (k-step g of 16 keys, 32-column block nb): two
+    // transposing reads, kAhead fragments ahead of its MFMA (2, 4, 6: within
+    // 1 % of each other)
+    constexpr int kAhead = 2;
+    u32x2 vd[kAhead + 1][2];
+    unsigned vofs_nb[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+        vofs_nb[nb] = (unsigned)((4 * hh + tr_s) * 256 + vsub) +
+                      ((((unsigned)(4 * nb) | vcl) ^ vs) << 4);
+    auto read_vd = [&](auto j_tag, const unsigned (&vad)[4]) {
+        constexpr int j = decltype(j_tag)::value, g = j / 4, nb = j % 4;
+        vd[j % (kAhead + 1)][0] = lds_tr16<16 * g * 256>(vad[nb]);
+        vd[j % (kAhead + 1)][1] = lds_tr16<(16 * g + 8) * 256>(vad[nb]);
+    };
+    // MFMA j of the pending product, after the wait that leaves the newer
+    // fragments' reads in flight
+    auto pv_step = [&](auto j_tag) {
+        constexpr int j = decltype(j_tag)::value, g = j / 4, nb = j % 4;
+        constexpr int newer = j + kAhead < 16 ? kAhead - 1 : 15 - j;
+        u32x2& a0 = vd[j % (kAhead + 1)][0];
+        u32x2& a1 = vd[j % (kAhead + 1)][1];
+        lgkm_wait_n<2 * newer>(a0, a1);
+        const u32x4 va = {a0[0], a0[1], a1[0], a1[1]};
+        o[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va),
+                                                        __builtin_bit_cast(bf16x8, pd[g]), o[nb], 0,
+                                                        0, 0);
+    };
+    auto v_addr = [&](const unsigned char* v_tile, unsigned (&vad)[4]) {
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) vad[nb] = (unsigned)(uintptr_t)v_tile + vofs_nb[nb];
+    };
+    auto compute_tile = [&](int t, const unsigned char* ks_lds, const unsigned char* v_prev,
+                            auto&& between, auto&& after) {
         const unsigned kbase = (unsigned)(uintptr_t)ks_lds + (unsigned)(lq * 256);
+        unsigned vad[4];
+        v_addr(v_prev, vad);
         f32x16 s0, s1;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             s0[v] = 0.f;
             s1[v] = 0.f;
         }
-        // S^T = K Q^T; K fragments are read two k-steps ahead of their MFMAs
-        // (lgkmcnt(2) leaves the newest pair in flight).
         u32x4 ka[3], kb[3];
-        // MFMA sections run at raised wave priority: when both waves of a
-        // SIMD are ready, the one feeding the matrix core issues first and
-        // the other's softmax VALU work fills the gaps.
-        __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             const unsigned ad = kbase + ((((unsigned)(2 * ks + hh)) ^ kswz) << 4);
@@ -859,50 +904,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
             const int cur = ks % 3;
-            if (ks + 1 < 8)
-                lgkm_wait2_keep2(ka[cur], kb[cur]);
-            else
-                lgkm_wait2(ka[cur], kb[cur]);
+            // behind them: the next K fragments, then V fragment 0
+            lgkm_wait2_keep2(ka[cur], kb[cur]);
             if (ks + 2 < 8) {
                 const int nx = (ks + 2) % 3;
                 const unsigned ad = kbase + ((((unsigned)(2 * (ks + 2) + hh)) ^ kswz) << 4);
                 ka[nx] = lds_b128<0>(ad);
                 kb[nx] = lds_b128<32 * 256>(ad);
             }
+            if (ks == 6) read_vd(std::integral_constant<int, 0>{}, vad);
+            if (ks == 7) read_vd(std::integral_constant<int, 1>{}, vad);
             s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ka[cur]),
                                                          qf[ks], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kb[cur]),
                                                          qf[ks], s1, 0, 0, 0);
             between(ks);
         }
+        __builtin_amdgcn_s_setprio(1);
 
-        __builtin_amdgcn_s_setprio(0);
-
-        // O^T += V^T P^T reads V^T fragments with transposing LDS reads of
-        // rows 16g + 4hh + s and +8 (row offsets 16g*256 and 8*256 are
-        // immediates): 8 reads per 32-column block nb, in two groups of 4
-        // that feed 2 MFMAs each. Block 0 is read now, ahead of the softmax;
-        // each later group is read one block ahead of its MFMAs.
-        const unsigned vbase = (unsigned)(uintptr_t)vt_lds + (unsigned)((4 * hh + tr_s) * 256 + vsub);
-        auto vaddr = [&](int nb) { return vbase + ((((unsigned)(4 * nb) | vcl) ^ vs) << 4); };
-        u32x2 vr[2][8];
-        auto read_v = [&](u32x2* d, int nb, int half) {
-            const unsigned ad = vaddr(nb);
-            if (half == 0) {
-                d[0] = lds_tr16<0>(ad);
-                d[1] = lds_tr16<8 * 256>(ad);
-                d[2] = lds_tr16<16 * 256>(ad);
-                d[3] = lds_tr16<24 * 256>(ad);
-            } else {
-                d[4] = lds_tr16<32 * 256>(ad);
-                d[5] = lds_tr16<40 * 256>(ad);
-                d[6] = lds_tr16<48 * 256>(ad);
-                d[7] = lds_tr16<56 * 256>(ad);
-            }
-        };
-        read_v(vr[0], 0, 0);
-        read_v(vr[0], 0, 1);
-
+        after();
         float s[32];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
@@ -911,9 +931,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
         }
         const int left = nkeys - t * kBf16BlockKeys;
         if (left < kBf16BlockKeys) {
-            // s[v] holds key kc(v) + 4*hh of the tile, kc(v) a compile-time
-            // constant: comparing kc(v) with lim - 4*hh keeps the per-lane
-            // key indices out of registers.
             const int lim = left - 4 * hh;
 #pragma unroll
             for (int v = 0; v < 32; ++v) {
@@ -921,35 +938,41 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
                 if (kc >= lim) s[v] = -INFINITY;
             }
         }
-
-        // Exponentiate against the running max; only when the tile's row sum
-        // overflows the bound (first tile, where the running max is -inf, or
-        // scores that grew far beyond it) take the slow path: raise the max
-        // to the tile max, rescale O and l, and exponentiate again.
-        // The tile's row sum comes from the matrix core (rsel above), so
-        // the VALU work per score is one FMA, one exponential and half a
-        // bf16 pack. (A 0 x inf product in that sum, from an infinite
-        // exponential, yields NaN, which fails the bound check as the inf
-        // itself would.)
-        bf16x8 pb[4];
-        auto exp_tile = [&](float mref) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-#pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    const float e0 = fast_exp2(fmaf(s[8 * g + i], cl2, -mref));
-                    const float e1 = fast_exp2(fmaf(s[8 * g + i + 1], cl2, -mref));
-                    pb[g][i] = (__bf16)e0;
-                    pb[g][i + 1] = (__bf16)e1;
-                }
-            }
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rsel, pb[g], acc, 0, 0, 0);
-            return rs_hi ? acc[1] : acc[0];
+        // Score pair e (0..15), of P fragment e / 4: FMAs at MFMA e of the
+        // pending product, exponentials at the next one, pack at MFMA e + kPack,
+        // when the product is done with the fragment it replaces (at most
+        // e + 3).
+        float x0[16], x1[16];
+        f32x4 rs = {0.f, 0.f, 0.f, 0.f};
+        auto pack = [&](int e) {
+            bf16x2 w;
+            w[0] = (__bf16)x0[e];
+            w[1] = (__bf16)x1[e];
+            pd[e / 4][e % 4] = __builtin_bit_cast(unsigned, w);
         };
-        float tot = exp_tile(m_run);
+        constexpr int kPack = 5;
+        static_for<16 + kPack>([&](auto mc) __attribute__((always_inline)) {
+            constexpr int m = decltype(mc)::value;
+            if constexpr (m < 16) {
+                pv_step(mc);
+                if constexpr (m + kAhead < 16)
+                    read_vd(std::integral_constant<int, m + kAhead>{}, vad);
+                x0[m] = fmaf(s[2 * m], cl2, -m_run);
+                x1[m] = fmaf(s[2 * m + 1], cl2, -m_run);
+            }
+            if constexpr (m >= 1 && m <= 16) {
+                x0[m - 1] = fast_exp2(x0[m - 1]);
+                x1[m - 1] = fast_exp2(x1[m - 1]);
+            }
+            if constexpr (m >= kPack) {
+                pack(m - kPack);
+                if constexpr ((m - kPack) % 4 == 3)
+                    rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        rsel, __builtin_bit_cast(bf16x8, pd[(m - kPack) / 4]), rs, 0, 0, 0);
+            }
+            if constexpr (m < 16) __builtin_amdgcn_sched_barrier(0);
+        });
+        float tot = rs_hi ? rs[1] : rs[0];
         if (__builtin_amdgcn_ballot_w64(!(tot <= kRowSumLimit))) {
             float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
 #pragma unroll
@@ -965,41 +988,40 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o[nb][v] *= corr;
             m_run = m_new;
-            tot = exp_tile(m_run);
+            rs = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    x0[4 * g + i] = fast_exp2(fmaf(s[8 * g + 2 * i], cl2, -m_run));
+                    x1[4 * g + i] = fast_exp2(fmaf(s[8 * g + 2 * i + 1], cl2, -m_run));
+                    pack(4 * g + i);
+                }
+                rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    rsel, __builtin_bit_cast(bf16x8, pd[g]), rs, 0, 0, 0);
+            }
+            tot = rs_hi ? rs[1] : rs[0];
         }
         l_run += tot;
-
-        // LDS reads complete in issue order, so lgkmcnt(4) waits for the
-        // older of the two groups in flight.
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            u32x2* cur = vr[nb & 1];
-            u32x2* nxt = vr[(nb + 1) & 1];
-            lgkm_wait_tr_n<4>(cur[0], cur[1], cur[2], cur[3]);
-            if (nb < 3) read_v(nxt, nb + 1, 0);
-            const u32x4 va0 = {cur[0][0], cur[0][1], cur[1][0], cur[1][1]};
-            const u32x4 va1 = {cur[2][0], cur[2][1], cur[3][0], cur[3][1]};
-            o[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va0), pb[0],
-                                                            o[nb], 0, 0, 0);
-            o[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va1), pb[1],
-                                                            o[nb], 0, 0, 0);
-            if (nb < 3) {
-                lgkm_wait_tr_n<4>(cur[4], cur[5], cur[6], cur[7]);
-                read_v(nxt, nb + 1, 1);
-            } else {
-                lgkm_wait_tr_n<0>(cur[4], cur[5], cur[6], cur[7]);
-            }
-            const u32x4 va2 = {cur[4][0], cur[4][1], cur[5][0], cur[5][1]};
-            const u32x4 va3 = {cur[6][0], cur[6][1], cur[7][0], cur[7][1]};
-            o[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va2), pb[2],
-                                                            o[nb], 0, 0, 0);
-            o[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va3), pb[3],
-                                                            o[nb], 0, 0, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
+    };
+    auto pv_last = [&](const unsigned char* v_prev) {
+        unsigned vad[4];
+        v_addr(v_prev, vad);
+        static_for<kAhead>([&](auto j) __attribute__((always_inline)) { read_vd(j, vad); });
+        static_for<16>([&](auto mc) __attribute__((always_inline)) {
+            constexpr int m = decltype(mc)::value;
+            pv_step(mc);
+            if constexpr (m + kAhead < 16) read_vd(std::integral_constant<int, m + kAhead>{}, vad);
+        });
     };
 
+    // V stage of step t (t % kVStages) and byte offset of that d steps on
+    int v3 = 0;
+    auto v_next = [&](int v) { return v + 1 == kVStages ? 0 : v + 1; };
+    auto v_of = [&](int v, int d) {
+        const int n = v + d;
+        return (n >= kVStages ? n - kVStages : n) * kBf16TileBytes;
+    };
     unsigned hw_next = ~0u;  // map words of the tile after the next one
     // first key of the next map load's tile, byte offset of the next
     // prep_tile's tile
@@ -1134,21 +1156,22 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
         if (ntiles > 0) {
             const unsigned g0 = load_gd(0);
             const unsigned g1 = load_gd(1);
-            prep_gd(tix(0), kv_next, gd_key, k_lds0, v_lds0, g0);
+            prep_gd(tix(0), kv_next, gd_key, k_lds, v_lds, g0);
             kv_next = next_off(kv_next, 0, kv_step, kv_wrap);
             gd_key = next_off(gd_key, 0, key_step, key_wrap);
 #pragma unroll
             for (int i = 0; i < 4; ++i) copy_gd(i);
             overwrite_gd();
-            prep_gd(tix(1), kv_next, gd_key, k_lds1, v_lds1, g1);
+            prep_gd(tix(1), kv_next, gd_key, k_lds + kBf16TileBytes, v_lds + kBf16TileBytes, g1);
             kv_next = next_off(kv_next, 1, kv_step, kv_wrap);
             gd_key = next_off(gd_key, 1, key_step, key_wrap);
             gd_next = load_gd(2);
         }
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_waitcnt(0);
         for (int t = 0; t < ntiles; ++t) {
-            unsigned char* kcur = (t & 1) ? k_lds1 : k_lds0;
-            unsigned char* vcur = (t & 1) ? v_lds1 : v_lds0;
+            unsigned char* kcur = k_lds + (t & 1) * kBf16TileBytes;
+            // V of step t - 1 (pending product); step t + 2's goes there next
+            unsigned char* vprev = v_lds + v_of(v3, 2);
             // The newest vector-memory operation of the wave is the
             // descriptor load issued at the end of the previous step (used
             // one step later); everything before it -- this tile's copies and
@@ -1159,15 +1182,16 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             wait_vm<1>();
             wg_barrier();
             if (active) {
-                compute_tile(tix(t), kcur, vcur, [&](int ks) {
+                compute_tile(tix(t), kcur, vprev, [&](int ks) {
                     if ((ks & 1) == 0) copy_gd(ks >> 1);
-                });
+                }, [] {});
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) copy_gd(i);
             }
             overwrite_gd();
-            prep_gd(tix(t + 2), kv_next, gd_key, kcur, vcur, gd_next);
+            prep_gd(tix(t + 2), kv_next, gd_key, kcur, vprev, gd_next);
+            v3 = v_next(v3);
             kv_next = next_off(kv_next, t + 2, kv_step, kv_wrap);
             gd_key = next_off(gd_key, t + 2, key_step, key_wrap);
             gd_next = load_gd(t + 3);
@@ -1179,24 +1203,23 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             map_next = next_off(map_next, 1, key_step, key_wrap);
             unsigned md[4] = {~0u, ~0u, ~0u, ~0u};
             decode_map(tix(0), hw0, md);
-            prep_tile(0, kv_next, k_lds0, v_lds0);
+            prep_tile(0, kv_next, k_lds, v_lds);
             kv_next = next_off(kv_next, 0, kv_step, kv_wrap);
 #pragma unroll
             for (int i = 0; i < 4; ++i) copy_pair(i, md);
         }
         // Compiler-visible wait for every load so far (Q, map, tile 0): the
         // loop then never waits for vector memory on the Q registers' account.
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_waitcnt(0);
         for (int t = 0; t < ntiles; ++t) {
-            // t counts loop steps; step t computes tile tix(t). Step t's tile
-            // lives in stage t & 1; step t+1's tile streams into the other
-            // stage, which held step t-1's: every wave finished reading it
-            // before it reached the barrier below, so one barrier per tile
-            // suffices
-            unsigned char* kcur = (t & 1) ? k_lds1 : k_lds0;
-            unsigned char* vcur = (t & 1) ? v_lds1 : v_lds0;
-            unsigned char* knext = (t & 1) ? k_lds0 : k_lds1;
-            unsigned char* vnext = (t & 1) ? v_lds0 : v_lds1;
+            // t counts loop steps; step t computes tile tix(t). Step t's K tile
+            // lives in stage t & 1, its V tile in stage t % 3; step t+1's
+            // tile streams into the next stage, which held a tile that every
+            // wave finished reading before it reached the barrier below, so
+            // one barrier per tile suffices
+            unsigned char* kcur = k_lds + (t & 1) * kBf16TileBytes;
+            unsigned char* knext = k_lds + ((t + 1) & 1) * kBf16TileBytes;
+            unsigned char* vnext = v_lds + v_of(v3, 1);
             // each wave's copies of step t's tile (and its map load) have
             // landed, then the barrier publishes the whole tile
             wait_vm<0>();
@@ -1213,26 +1236,32 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             decode_map(tix(t + 1), hw1, md);
             prep_tile(t + 1, kv_next, knext, vnext);
             kv_next = next_off(kv_next, t + 1, kv_step, kv_wrap);
-            // wave-uniform: the group mixes arena and original rows, each
-            // row's source chosen per lane (copy_pair)
+            // wave-uniform: the group mixes arena and original rows. Its arena
+            // rows go out after the copies of the original ones and replace
+            // them (a wave's vector-memory operations complete in issue order).
             const bool mixed = kMap && grp_mapped && !(kRuns && grp_run);
+            auto overwrite = [&] {
+                if (__builtin_expect(!mixed, 1)) return;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (md[i] != ~0u) copy_pair(i, md);
+            };
             if (active) {
-                if (__builtin_expect(mixed, 0)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) copy_pair(i, md);
-                }
-                compute_tile(tix(t), kcur, vcur, [&](int ks) {
-                    if ((ks & 1) == 0) copy_plain(ks >> 1);
-                });
-            } else if (mixed) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) copy_pair(i, md);
+                compute_tile(
+                    tix(t), kcur, v_lds + v_of(v3, 2),
+                    [&](int ks) {
+                        if ((ks & 1) == 0) copy_plain(ks >> 1);
+                    },
+                    overwrite);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) copy_plain(i);
+                overwrite();
             }
+            v3 = v_next(v3);
         }
     }
+    if (active && ntiles > 0) pv_last(v_lds + v_of(v3, 2));
     // the trailing copies land before the workgroup's LDS is released, and
     // every wave has read its last tile before the epilogue stages output
     // rows there
@@ -1240,11 +1269,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     wg_barrier();
     if (!active) return;
 
-    // Stage in the last tile's stage: every wave has passed the barrier
-    // after its last read, and the trailing copies target the other stage.
-    unsigned char* last_k = (ntiles > 0 && ((ntiles - 1) & 1)) ? k_lds1 : k_lds0;
-    unsigned char* last_v = (ntiles > 0 && ((ntiles - 1) & 1)) ? v_lds1 : v_lds0;
-    unsigned char* stage = (wave < 2 ? last_k : last_v) + 8192 * (wave & 1);
+    // Every copy has landed and every tile has been read (barrier above): the
+    // output rows are staged in the K stages.
+    unsigned char* stage = k_lds + 8192 * wave;
     if (a.splits > 1)
         store_rows_staged<_Float16, true>(a, c, wave, lane, o, m_run, l_run, stage);
     else
