@@ -100,6 +100,23 @@ def test_proj_gemm_rejects_unsupported_shapes(lib):
     (129, 32, 128, True, False), (1560, 1536, 1536, False, True), (300, 1536, 384, True, True),
 ])
 def test_fp32_linear_tiled(rows, K, N, acc, bias):
+    _check_fp32_linear(rows, K, N, acc, bias)
+
+
+# short inner dimension: every K of the register kernel and its neighbours on
+# the general one, rows around a wave's 16 and a block's 64, features around
+# the block's 256 and a multiple of 4 or not
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N,acc,bias", [
+    (1, 4, 4, False, True), (15, 8, 252, False, False), (17, 12, 256, True, True),
+    (65, 16, 260, False, True), (1560, 16, 1536, False, True), (63, 16, 258, True, True),
+    (129, 20, 256, False, True), (64, 15, 256, False, True), (64, 16, 1024, True, False),
+])
+def test_fp32_linear_short_inner(rows, K, N, acc, bias):
+    _check_fp32_linear(rows, K, N, acc, bias)
+
+
+def _check_fp32_linear(rows, K, N, acc, bias):
     print(f"fp32 linear rows={rows} K={K} N={N} acc={acc}", flush=True)
     rng = np.random.default_rng(rows + K + N)
     x = rng.standard_normal((rows, K)).astype(np.float32)
