@@ -789,8 +789,9 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GenericArgs a) {
 // Short inner dimension (K = 4, 8, 12 or 16), fp32: y (+)= x W^T + b.
 //
 // A lane keeps the K weights of 4 neighbouring features in registers (through
-// LDS: loaded directly, 64 lines per load, they took 15 us more) and its wave walks kThinRows rows, whose values are wave-uniform (scalar loads), so a
-// row costs 4 K FMAs and one 16-byte store per lane: bound by writing y. The
+// LDS: loaded directly, 64 lines per load, the kernel took 37 us) and its wave
+// walks kThinRows rows, whose values are wave-uniform (scalar loads), so a row
+// costs 4 K FMAs and one 16-byte store per lane: bound by writing y. The
 // 64 x 64 tiles of gemm_generic_kernel pad K to 32 and stage both operands
 // through LDS for one chunk of work. 12480 rows x 16 -> 1536 features:
 // 51 -> 32 us (2.4 TB/s written). 8 rows per wave 32.6 us, 32 rows 38.7.
