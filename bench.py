@@ -368,10 +368,11 @@ def motion_bench(args, torch, stream):
     the 30 x 52 cell means and the 98 tile change rates per pair.
 
     Whole clip: W warmup, K timed runs (HIP events on the launch stream).
-    Per launch: one run of kvp_farneback_profile (an event after every
-    launch); the kind with the most time at level 0 is the dominant kernel,
-    its achieved bandwidth = algorithmic bytes of one level-0 pass over the
-    clip / the average duration of its passes."""
+    Per pass over the clip (a kernel, level and iteration): one run of
+    kvp_farneback_profile (an event after every launch); the kind with the
+    most time at level 0 is the dominant kernel, its achieved bandwidth =
+    algorithmic bytes of one level-0 pass / the average duration of its
+    passes."""
     from kvpersist import motion, workloads
 
     n, H, W = args.motion_frames, 480, 832
@@ -395,9 +396,9 @@ def motion_bench(args, torch, stream):
     clip_ms = e0.elapsed_time(e1) / args.steps
     finite = bool(torch.isfinite(change).all())
 
-    _, launches = motion.farneback_profile(clip, flows, stream=stream)
+    _, steps = motion.farneback_profile(clip, flows, stream=stream)
     per_kind, lvl0 = {}, {}
-    for kind, level, ms in launches:
+    for kind, level, ms in steps:
         per_kind[kind] = per_kind.get(kind, 0.0) + ms
         if level == 0:
             lvl0.setdefault(kind, []).append(ms)
@@ -405,16 +406,14 @@ def motion_bench(args, torch, stream):
     P, pairs = H * W, n - 1
 
     def level0_roof(kind):
-        # a level-0 pass over the clip may be several launches (chunks of pairs)
         units = n if kind in MOTION_PER_FRAME else pairs
-        passes = motion.FARNEBACK["iterations"] if kind == "box_flow" else 1
+        passes = len(lvl0[kind])
         nbytes = MOTION_BYTES_PER_PX[kind] * P * units
         ms = sum(lvl0[kind]) / passes
         ach = nbytes / (ms * 1e-3) / 1e9
         return {"bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4), "avg_pass_ms": round(ms, 5),
-                "passes_per_clip": passes, "launches_per_clip": len(lvl0[kind]),
-                "bytes_per_pass": nbytes,
+                "passes_per_clip": passes, "bytes_per_pass": nbytes,
                 "per_pass": f"{MOTION_BYTES_PER_PX[kind]} B/px x {P} px x {units} "
                             f"{'frames' if kind in MOTION_PER_FRAME else 'pairs'}"}
 
@@ -441,7 +440,7 @@ def motion_bench(args, torch, stream):
                                f"for all {pairs} pairs, 30x52 cells, 98 tiles of 16",
                    "frames": n, "dtype": "f32"},
         "launch_ms_per_clip": {k: round(v, 4) for k, v in per_kind.items()},
-        "launches_per_clip": len(launches),
+        "passes_per_clip": len(steps),
         "roofline": dict(level0_roof(dominant), kernel=dominant, traffic=traffic),
         "level0_rooflines": {k: level0_roof(k) for k in lvl0},
     }

@@ -1173,13 +1173,21 @@ int check_params(int nf, int W, int H, double pyr_scale, int levels, int winsize
     return 0;
 }
 
-// Launch timeline for kvp_farneback_profile: an event after every launch.
+// Launch timeline for kvp_farneback_profile: an event after every launch. A step
+// is one kernel's work of one level and iteration; a clip taken in chunks makes
+// several launches of a step, which share its entry, so that the entries of a
+// clip do not grow with its length.
 struct Timeline {
+    struct Step {
+        int kind, level, iteration;
+        float ms;
+    };
     hipStream_t st;
-    std::vector<hipEvent_t> ev;
-    std::vector<int> kind, level;
+    std::vector<hipEvent_t> ev;  // the first one before the first launch
+    std::vector<size_t> step_of;  // of launch i, between events i and i + 1
+    std::vector<Step> steps;
     bool ok = true;
-    void mark(int k, int lv) {
+    void record() {
         hipEvent_t e;
         if (hipEventCreate(&e) != hipSuccess) {
             ok = false;
@@ -1187,8 +1195,25 @@ struct Timeline {
         }
         if (hipEventRecord(e, st) != hipSuccess) ok = false;
         ev.push_back(e);
-        kind.push_back(k);
-        level.push_back(lv);
+    }
+    void launched(int kind, int level, int iteration) {
+        record();
+        size_t i = 0;
+        while (i < steps.size() && !(steps[i].kind == kind && steps[i].level == level &&
+                                     steps[i].iteration == iteration))
+            ++i;
+        if (i == steps.size()) steps.push_back({kind, level, iteration, 0.f});
+        step_of.push_back(i);
+    }
+    // waits for the launches and sums their times; false if an event failed
+    bool sum() {
+        if (!ok || ev.empty() || hipEventSynchronize(ev.back()) != hipSuccess) return false;
+        for (size_t i = 0; i < step_of.size(); ++i) {
+            float ms = 0.f;
+            if (hipEventElapsedTime(&ms, ev[i], ev[i + 1]) != hipSuccess) return false;
+            steps[step_of[i]].ms += ms;
+        }
+        return true;
     }
     ~Timeline() {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);
@@ -1231,10 +1256,10 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
     const int m = winsize / 2;
     const double box_scale = 1.0 / ((double)winsize * winsize);
 
-    auto mark = [&](int kind, int lv) {
-        if (tl) tl->mark(kind, lv);
+    auto mark = [&](int kind, int lv, int iteration = 0) {
+        if (tl) tl->launched(kind, lv, iteration);
     };
-    mark(-1, -1);
+    if (tl) tl->record();
 
     // Image and expansion of frames [f0, f0 + n) on plan levels [l0, l1), as
     // one launch each (more only past kPyrLevels levels or kPyrTaps taps).
@@ -1359,7 +1384,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
                     flow_step_kernel<true><<<grid, kFsThreads, 0, st>>>(a);
                 else
                     flow_step_kernel<false><<<grid, kFsThreads, 0, st>>>(a);
-                mark(KIND_FLOW, l.k);
+                mark(KIND_FLOW, l.k, it);
             }
             return launch_ok("farneback iterations");
         }
@@ -1378,14 +1403,14 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
         const dim3 box_grid(strips, (l.h + rows - 1) / rows, n);
         for (int it = 0; it < iterations; ++it) {
             update_matrices_kernel<<<pix, 256, 0, st>>>(a, M);
-            mark(KIND_MATRICES, l.k);
+            mark(KIND_MATRICES, l.k, it);
             if (narrow)
                 update_flow_kernel<128><<<box_grid, 128, 0, st>>>(M, l.w, l.h, m, rows, box_scale,
                                                                    fl);
             else
                 update_flow_kernel<256><<<box_grid, 256, 0, st>>>(M, l.w, l.h, m, rows, box_scale,
                                                                    fl);
-            mark(KIND_FLOW, l.k);
+            mark(KIND_FLOW, l.k, it);
         }
         return launch_ok("farneback iterations");
     };
@@ -1456,29 +1481,20 @@ int kvp_farneback_profile(const unsigned char* frames, int num_frames, int width
                                        poly_sigma, flags, workspace, workspace_bytes, flows,
                                        stream, &tl);
     if (rc) return rc;
-    if (!tl.ok || tl.ev.empty()) {
-        kvp::set_error("farneback_profile: event creation failed");
+    if (!tl.sum()) {
+        kvp::set_error("farneback_profile: event timing failed");
         return 1;
     }
-    if (hipEventSynchronize(tl.ev.back()) != hipSuccess) {
-        kvp::set_error("farneback_profile: event synchronize failed");
-        return 1;
-    }
-    const int n = (int)tl.ev.size() - 1;
+    const int n = (int)tl.steps.size();
     *count = n;
     if (n > capacity) {
-        kvp::set_error("farneback_profile: %d launches > capacity %d", n, capacity);
+        kvp::set_error("farneback_profile: %d steps > capacity %d", n, capacity);
         return 1;
     }
     for (int i = 0; i < n; ++i) {
-        float ms = 0.f;
-        if (hipEventElapsedTime(&ms, tl.ev[i], tl.ev[i + 1]) != hipSuccess) {
-            kvp::set_error("farneback_profile: elapsed time unavailable");
-            return 1;
-        }
-        launch_ms[i] = ms;
-        launch_kind[i] = tl.kind[i + 1];
-        launch_level[i] = tl.level[i + 1];
+        launch_ms[i] = tl.steps[i].ms;
+        launch_kind[i] = tl.steps[i].kind;
+        launch_level[i] = tl.steps[i].level;
     }
     return 0;
 }

@@ -105,7 +105,9 @@ KINDS = ("blur_rows", "blur_cols_resize", "poly_exp", "matrices_init", "box_flow
 def farneback_profile(frames, flows: torch.Tensor | None = None, stream: int | None = None,
                       **params):
     """farneback_flows with an event after every launch (synchronises):
-    -> (flows, [(kind name, pyramid level, ms), ...] in launch order)."""
+    -> (flows, [(kind name, pyramid level, ms), ...] in launch order), one entry for
+    each kernel, level and iteration; the launches that a long clip's chunks of pairs
+    take of it are summed."""
     fr = _frames_u8(frames)
     n, H, W = fr.shape
     p = _params(params)

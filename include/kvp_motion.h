@@ -57,14 +57,18 @@ int kvp_farneback_flow(const unsigned char* prev, const unsigned char* next,
                        long workspace_bytes, void* stream);
 
 /* kvp_farneback_flows with an event after every kernel launch, for
- * measurement (no counterpart in the reference, whose flow is a cv2 call):
- * launch i took launch_ms[i] on `stream`; launch_kind[i] is 1 pre-blur +
+ * measurement (no counterpart in the reference, whose flow is a cv2 call).
+ * Entry i is one step: a kernel's work on one level (and, of the iterations'
+ * kernels, one iteration) for the whole clip, in the order of the first
+ * launches. Long clips take a step in several launches, chunks of pairs; their
+ * times are summed, so the number of entries does not grow with the clip.
+ * Step i took launch_ms[i] on `stream`; launch_kind[i] is 1 pre-blur +
  * resize, 2 polynomial expansion, 3 initial flow of a level, 4 flow (a whole
  * iteration for window sizes 14 and 15; otherwise box filter + solve), 5 matrix
  * update (other window sizes); 0 is not used. launch_level[i] is the pyramid
- * level (0 = full size), the lowest one of a launch that covers several; a
- * level's pairs may be taken in several launches. Synchronises the
- * stream. *count receives the number of launches (an error if > capacity). */
+ * level (0 = full size), the lowest one of a step that covers several.
+ * Synchronises the stream. *count receives the number of entries (an error if
+ * > capacity). */
 int kvp_farneback_profile(const unsigned char* frames, int num_frames,
                           int width, int height, double pyr_scale, int levels,
                           int winsize, int iterations, int poly_n,

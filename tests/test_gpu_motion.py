@@ -352,3 +352,17 @@ def test_pyramid_and_strip_edges_match_oracle(H, W, params):
     clip = workloads.synthetic_clip(2, H, W, seed=H)
     got = motion.calc_optical_flow_farneback(clip[0], clip[1], **params).cpu().numpy()
     _flow_ok(got, fb.calc_optical_flow_farneback(clip[0], clip[1], **params), f"{H}x{W} {params}")
+
+
+def _steps(frames, H, W, **params):
+    clip = torch.from_numpy(workloads.synthetic_clip(frames, H, W, seed=frames)).to(DEV)
+    flows, steps = motion.farneback_profile(clip, **params)
+    assert torch.equal(flows, motion.farneback_flows(clip, **params))
+    assert all(ms > 0 for _, _, ms in steps)
+    return [(kind, level) for kind, level, _ in steps]
+
+
+@pytest.mark.parametrize("params", [{}, dict(winsize=9)])
+def test_profile_entries_do_not_grow_with_the_clip(params):
+    """20 and 60 frames of 832x480 take 2 and 4 chunks of the full-size level's pairs."""
+    assert _steps(20, 480, 832, **params) == _steps(60, 480, 832, **params)
