@@ -360,6 +360,32 @@ MOTION_BYTES_PER_PX = {
 MOTION_PER_FRAME = ("poly_exp",)
 
 
+def motion_level0(steps, frames, pixels):
+    """Rates of the full-size level's passes over a clip, by kind: steps as
+    motion.farneback_profile returns them. A step that covers several levels (a
+    short clip's expansion) is no level-0 pass, and a kind without a byte model
+    has no rate."""
+    alone = all(level == 0 for _, level, _ in steps) or any(
+        kind == "poly_exp" and level > 0 for kind, level, _ in steps)
+    lvl0 = {}
+    for kind, level, ms in steps:
+        if level == 0 and kind in MOTION_BYTES_PER_PX and (alone or kind != "poly_exp"):
+            lvl0.setdefault(kind, []).append(ms)
+    roofs = {}
+    for kind, times in lvl0.items():
+        units = frames if kind in MOTION_PER_FRAME else frames - 1
+        nbytes = MOTION_BYTES_PER_PX[kind] * pixels * units
+        ms = sum(times) / len(times)
+        ach = nbytes / (ms * 1e-3) / 1e9
+        roofs[kind] = {
+            "bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(ach / HBM_PEAK_GBS, 4), "avg_pass_ms": round(ms, 5),
+            "passes_per_clip": len(times), "bytes_per_pass": nbytes,
+            "per_pass": f"{MOTION_BYTES_PER_PX[kind]} B/px x {pixels} px x {units} "
+                        f"{'frames' if kind in MOTION_PER_FRAME else 'pairs'}"}
+    return roofs
+
+
 def motion_bench(args, torch, stream):
     """Upstream motion producer (reference: traces/gen_motion_from_video.py:
     104-121) over a synthetic clip resident in HBM: --motion-frames uint8 gray
@@ -397,25 +423,12 @@ def motion_bench(args, torch, stream):
     finite = bool(torch.isfinite(change).all())
 
     _, steps = motion.farneback_profile(clip, flows, stream=stream)
-    per_kind, lvl0 = {}, {}
-    for kind, level, ms in steps:
+    per_kind = {}
+    for kind, _, ms in steps:
         per_kind[kind] = per_kind.get(kind, 0.0) + ms
-        if level == 0:
-            lvl0.setdefault(kind, []).append(ms)
-    dominant = max(lvl0, key=lambda k: sum(lvl0[k]))
     P, pairs = H * W, n - 1
-
-    def level0_roof(kind):
-        units = n if kind in MOTION_PER_FRAME else pairs
-        passes = len(lvl0[kind])
-        nbytes = MOTION_BYTES_PER_PX[kind] * P * units
-        ms = sum(lvl0[kind]) / passes
-        ach = nbytes / (ms * 1e-3) / 1e9
-        return {"bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach / HBM_PEAK_GBS, 4), "avg_pass_ms": round(ms, 5),
-                "passes_per_clip": passes, "bytes_per_pass": nbytes,
-                "per_pass": f"{MOTION_BYTES_PER_PX[kind]} B/px x {P} px x {units} "
-                            f"{'frames' if kind in MOTION_PER_FRAME else 'pairs'}"}
+    roofs = motion_level0(steps, n, P)
+    dominant = max(roofs, key=lambda k: roofs[k]["avg_pass_ms"] * roofs[k]["passes_per_clip"])
 
     # fabric bytes of the level-0 launches from rocprofv3 FETCH_SIZE / WRITE_SIZE
     # runs of this workload, scaled by a copy-kernel calibration (committed)
@@ -441,8 +454,8 @@ def motion_bench(args, torch, stream):
                    "frames": n, "dtype": "f32"},
         "launch_ms_per_clip": {k: round(v, 4) for k, v in per_kind.items()},
         "passes_per_clip": len(steps),
-        "roofline": dict(level0_roof(dominant), kernel=dominant, traffic=traffic),
-        "level0_rooflines": {k: level0_roof(k) for k in lvl0},
+        "roofline": dict(roofs[dominant], kernel=dominant, traffic=traffic),
+        "level0_rooflines": roofs,
     }
     if not args.no_cpu_baseline:
         out["cpu_baseline"] = motion_cpu_baseline(clip[:3].cpu().numpy())

@@ -1275,7 +1275,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
             poly = blur;
             int blur_blocks = 0, poly_blocks = 0, taps = 0;
             size_t lds = 0;
-            int lo_level = plan[l0].k;
+            int blur_level = 0, lo_level = 0;  // the lowest level of each launch
             for (; l0 < l1 && poly.levels < kPyrLevels; ++l0) {
                 const Level& l = plan[l0];
                 if (l.k > 0 && taps + l.ksize > kPyrTaps) break;
@@ -1312,6 +1312,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
                     v.first_block = blur_blocks;
                     blur_blocks += v.tiles_x * ((l.h + v.tile_h - 1) / v.tile_h);
                     blur.lv[blur.levels++] = v;
+                    blur_level = l.k;
                 } else {
                     v.img = -1;
                 }
@@ -1324,7 +1325,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
             }
             if (blur_blocks) {
                 preblur_kernel<<<dim3(blur_blocks, 1, n), 256, lds, st>>>(blur);
-                mark(KIND_PREBLUR, lo_level);
+                mark(KIND_PREBLUR, blur_level);
             }
             if (poly_n == 5)
                 poly_exp_kernel<5><<<dim3(poly_blocks, 1, n), kPeThreads, 0, st>>>(poly, pt);

@@ -366,3 +366,14 @@ def _steps(frames, H, W, **params):
 def test_profile_entries_do_not_grow_with_the_clip(params):
     """20 and 60 frames of 832x480 take 2 and 4 chunks of the full-size level's pairs."""
     assert _steps(20, 480, 832, **params) == _steps(60, 480, 832, **params)
+
+
+def test_profile_levels():
+    """A step is labelled with the lowest level it covers: the pre-blur only ever
+    covers reduced levels, the expansion all of them where one chunk holds the
+    clip's pairs (2 frames) and the full-size level by itself where not (20)."""
+    flow = lambda lv, first: [(first, lv)] * (first is not None) + [(motion.KINDS[4], lv)] * 3
+    blur, expand, init = motion.KINDS[1:4]
+    coarse = flow(3, None) + flow(2, init) + flow(1, init)
+    assert _steps(2, 480, 832) == [(blur, 1), (expand, 0)] + coarse + flow(0, init)
+    assert _steps(20, 480, 832) == [(blur, 1), (expand, 1)] + coarse + [(expand, 0)] + flow(0, init)
