@@ -350,12 +350,12 @@ def producer_cpu_baseline(model, cfg, frames, layers):
 
 
 # Algorithmic HBM bytes per pixel of one full-size (level 0) pass, per frame
-# (expansion) or per pair (flow kinds); fp32 planes, uint8 frames. box_flow is
-# a whole iteration: flow and both frames' expansions in, flow out.
+# (expansion) or per pair (flow kinds); fp32 planes, uint8 frames. flow is a
+# whole iteration: flow and both frames' expansions in, flow out.
 MOTION_BYTES_PER_PX = {
     "poly_exp": 1 + 5 * 4,            # uint8 frame in, 5 expansion values out
-    "matrices_init": 2 + 2 * 4,       # coarse flow (1/4 px), initial flow out
-    "box_flow": 2 * 4 + 5 * 4 * 2 + 2 * 4,
+    "init_flow": 2 + 2 * 4,           # coarse flow (1/4 px), initial flow out
+    "flow": 2 * 4 + 5 * 4 * 2 + 2 * 4,
 }
 MOTION_PER_FRAME = ("poly_exp",)
 

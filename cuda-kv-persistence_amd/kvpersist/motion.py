@@ -99,7 +99,8 @@ def farneback_flows(frames, flows: torch.Tensor | None = None, stream: int | Non
     return flows
 
 
-KINDS = ("blur_rows", "blur_cols_resize", "poly_exp", "matrices_init", "box_flow", "matrices")
+# names of launch_kind (include/kvp_motion.h); 0 is not used
+KINDS = ("", "preblur", "poly_exp", "init_flow", "flow", "matrices")
 
 
 def farneback_profile(frames, flows: torch.Tensor | None = None, stream: int | None = None,

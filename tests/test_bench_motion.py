@@ -36,3 +36,8 @@ def test_only_passes_of_the_full_size_level_alone_are_rated(merged):
 def test_one_level_is_rated_alone():
     roofs = bench.motion_level0([(EXPAND, 0, 1.0), (FLOW, 0, 1.0)], 2, 1000)
     assert set(roofs) == {EXPAND, FLOW}
+
+
+def test_kind_names_are_those_of_the_launches_that_exist():
+    assert motion.KINDS == ("", "preblur", "poly_exp", "init_flow", "flow", "matrices")
+    assert set(bench.MOTION_BYTES_PER_PX) < set(motion.KINDS)
