@@ -26,6 +26,8 @@ import argparse
 import csv
 import json
 import sys
+import threading
+from collections import OrderedDict
 from dataclasses import dataclass, field
 from datetime import date
 from pathlib import Path
@@ -40,19 +42,57 @@ from .api import _check, _ptr
 FARNEBACK = dict(pyr_scale=0.5, levels=3, winsize=15, iterations=3, poly_n=5, poly_sigma=1.2,
                  flags=0)
 
-# One workspace per device, shared by every call there: calls that overlap on
-# different streams of one device race on it.
-_workspaces: dict[int, torch.Tensor] = {}
+# Workspaces kept for reuse, by device and stream, per thread: calls on one stream
+# from one thread reuse its workspace in stream order. Calls that may overlap (on
+# different streams, or from two threads whose launches interleave on one stream)
+# never share one. A thread keeps the _MAX_WORKSPACES it used last, until it ends.
+_MAX_WORKSPACES = 8
+_STREAM_PER_THREAD = 2           # hipStreamPerThread: another stream in every thread
+_local = threading.local()
 
 
-def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Per-device workspace, grown on demand (calls on one device share it)."""
+def _torch_stream(device: torch.device, stream: int):
+    """The stream a raw handle stands for (0 and 1: the null stream)."""
+    if stream in (0, 1):
+        return torch.cuda.default_stream(device)
+    return torch.cuda.ExternalStream(stream, device=device)
+
+
+class _Workspace:
+    """Device bytes of one stream, from that stream's share of the allocator:
+    whoever gets the memory next runs behind the kernels that still use it. The
+    allocator cannot tell one thread's hipStreamPerThread from another's, so
+    memory used there changes hands only when the device is idle."""
+
+    def __init__(self, device: torch.device, stream: int, nbytes: int):
+        self.idle_device = device if stream == _STREAM_PER_THREAD else None
+        with torch.cuda.stream(_torch_stream(device, 0 if self.idle_device else stream)):
+            self.buf = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+        if self.idle_device:
+            torch.cuda.synchronize(device)
+
+    def __del__(self):
+        if getattr(self, "idle_device", None) and torch is not None:
+            torch.cuda.synchronize(self.idle_device)
+
+
+def _workspace(device: torch.device, stream: int | None, nbytes: int) -> torch.Tensor:
+    """This thread's workspace for calls on a stream of a device, grown on demand."""
+    if torch.cuda.is_current_stream_capturing():
+        # memory of the graph's own, which its replays keep
+        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    ws = _workspaces.get(idx)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        _workspaces[idx] = ws
-    return ws
+    stream = int(getattr(stream, "value", stream) or 0)
+    kept = getattr(_local, "workspaces", None)
+    if kept is None:
+        kept = _local.workspaces = OrderedDict()
+    ws = kept.pop((idx, stream), None)
+    if ws is None or ws.buf.numel() < nbytes:
+        ws = _Workspace(torch.device(device.type, idx), stream, nbytes)
+    kept[idx, stream] = ws
+    if len(kept) > _MAX_WORKSPACES:
+        kept.popitem(last=False)
+    return ws.buf
 
 
 def _frames_u8(x, device=None) -> torch.Tensor:
@@ -87,7 +127,7 @@ def farneback_flows(frames, flows: torch.Tensor | None = None, stream: int | Non
     need = lib.kvp_farneback_workspace_bytes(n, W, H, float(p["pyr_scale"]), int(p["levels"]))
     if need < 0:
         raise ValueError(f"bad clip shape {tuple(fr.shape)} or pyramid parameters {p}")
-    ws = _workspace(fr.device, need)
+    ws = _workspace(fr.device, stream, need)
     if flows is None:
         flows = torch.empty(n - 1, H, W, 2, dtype=torch.float32, device=fr.device)
     elif flows.shape != (n - 1, H, W, 2) or flows.dtype != torch.float32:
@@ -116,7 +156,7 @@ def farneback_profile(frames, flows: torch.Tensor | None = None, stream: int | N
     need = lib.kvp_farneback_workspace_bytes(n, W, H, float(p["pyr_scale"]), int(p["levels"]))
     if need < 0:
         raise ValueError(f"bad clip shape {tuple(fr.shape)} or pyramid parameters {p}")
-    ws = _workspace(fr.device, need)
+    ws = _workspace(fr.device, stream, need)
     if flows is None:
         flows = torch.empty(n - 1, H, W, 2, dtype=torch.float32, device=fr.device)
     cap = 1024
@@ -149,7 +189,7 @@ def calc_optical_flow_farneback(prev, next, flow=None, pyr_scale=0.5, levels=3, 
     need = lib.kvp_farneback_workspace_bytes(2, W, H, float(pyr_scale), int(levels))
     if need < 0:
         raise ValueError(f"bad frame size {W}x{H} or pyramid parameters")
-    ws = _workspace(a.device, need)
+    ws = _workspace(a.device, stream, need)
     if flow is None:
         flow = torch.empty(H, W, 2, dtype=torch.float32, device=a.device)
     _check(lib.kvp_farneback_flow(_ptr(a), _ptr(b), _ptr(flow), W, H, float(pyr_scale),

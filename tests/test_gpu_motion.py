@@ -15,6 +15,8 @@ the far-border band, the pair entry point equals the clip entry point bit
 for bit.
 """
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -377,3 +379,61 @@ def test_profile_levels():
     coarse = flow(3, None) + flow(2, init) + flow(1, init)
     assert _steps(2, 480, 832) == [(blur, 1), (expand, 0)] + coarse + flow(0, init)
     assert _steps(20, 480, 832) == [(blur, 1), (expand, 1)] + coarse + [(expand, 0)] + flow(0, init)
+
+
+def test_calls_overlapping_on_streams_and_threads_equal_serial_ones():
+    """Calls on two streams, and from two threads on one stream, each with its own
+    workspace; the second round outgrows it while the first is still in flight."""
+    clips = [torch.from_numpy(workloads.synthetic_clip(n, 240, 416, seed=n)).to(DEV)
+             for n in (6, 7, 24, 25)]
+    want = [motion.farneback_flows(c) for c in clips]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [torch.full_like(w, float("nan")) for w in want]
+    torch.cuda.synchronize()
+    for i, (c, o) in enumerate(zip(clips, outs)):
+        motion.farneback_flows(c, o, stream=streams[i % 2].cuda_stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+    for o in outs:
+        o.fill_(float("nan"))
+    torch.cuda.synchronize()
+
+    def work(k):
+        for c, o in list(zip(clips, outs))[k::2]:
+            motion.farneback_flows(c, o, stream=streams[0].cuda_stream)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
+def test_per_thread_stream():
+    clip = torch.from_numpy(workloads.synthetic_clip(3, 96, 128, seed=1)).to(DEV)
+    want = motion.farneback_flows(clip)
+    out = torch.full_like(want, float("nan"))
+    torch.cuda.synchronize()
+    motion.farneback_flows(clip, out, stream=2)      # hipStreamPerThread
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
+def test_captured_flow_replays_between_eager_calls():
+    a, b = (torch.from_numpy(workloads.synthetic_clip(4, 96, 128, seed=s)).to(DEV) for s in (1, 2))
+    want = motion.farneback_flows(a), motion.farneback_flows(b)
+    clip, out = a.clone(), torch.empty_like(want[0])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        motion.farneback_flows(clip, out, stream=torch.cuda.current_stream().cuda_stream)
+    for i in range(4):
+        clip.copy_((a, b)[i % 2])
+        out.fill_(float("nan"))
+        graph.replay()
+        eager = motion.farneback_flows((a, b)[1 - i % 2])
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i % 2]) and torch.equal(eager, want[1 - i % 2]), i

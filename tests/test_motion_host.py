@@ -4,8 +4,11 @@ CLI and the variance harness read (reference:
 traces/gen_motion_from_video.py:121-149, src/run_policy_experiment.cu:45-69)."""
 
 import csv
+import threading
 
 import numpy as np
+import pytest
+import torch
 
 from kvpersist import motion
 from oracle import farneback as fb
@@ -35,3 +38,46 @@ def test_csv_round_trip(tmp_path):
     assert s.shape == (5, 98) and s.dtype == np.float32
     want = np.array([[np.float32(f"{v:.6f}") for v in row] for row in change])
     assert np.array_equal(s, want)
+
+
+@pytest.fixture
+def on_host(monkeypatch):
+    """motion._workspace with host tensors in place of device memory."""
+    class Host:
+        def __init__(self, device, stream, nbytes):
+            self.buf = torch.empty(nbytes, dtype=torch.uint8)
+
+    monkeypatch.setattr(motion, "_Workspace", Host)
+    monkeypatch.setattr(motion, "_local", threading.local())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return torch.device("cuda", 0)
+
+
+def test_workspaces_are_kept_by_device_stream_and_thread(on_host):
+    def ws(stream, nbytes=64, device=on_host):
+        return motion._workspace(device, stream, nbytes)
+
+    a = ws(None)
+    assert ws(0) is a and ws(None, 10) is a      # the null stream, smaller calls
+    b = ws(0x1000)
+    assert b is not a and ws(0x1000) is b
+    assert ws(None, device=torch.device("cuda", 1)) is not a
+    grown = ws(0x1000, 128)
+    assert grown.numel() == 128 and ws(0x1000) is grown
+    other = []
+    t = threading.Thread(target=lambda: other.append(ws(0x1000)))
+    t.start()
+    t.join()
+    assert other[0] is not grown and ws(0x1000) is grown
+
+
+def test_a_thread_keeps_a_bounded_number_of_workspaces(on_host):
+    first = motion._workspace(on_host, 0x100, 1)
+    for i in range(2, 2 + motion._MAX_WORKSPACES - 1):
+        motion._workspace(on_host, 0x100 * i, 1)
+    assert motion._workspace(on_host, 0x100, 1) is first          # now the last used
+    kept = motion._local.workspaces
+    second = kept[0, 0x200].buf
+    motion._workspace(on_host, 0x10000, 1)
+    assert len(kept) == motion._MAX_WORKSPACES and (0, 0x200) not in kept
+    assert motion._workspace(on_host, 0x200, 1) is not second
