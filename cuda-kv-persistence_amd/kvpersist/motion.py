@@ -51,6 +51,10 @@ _STREAM_PER_THREAD = 2           # hipStreamPerThread: another stream in every t
 _local = threading.local()
 
 
+def _handle(stream) -> int:
+    return int(getattr(stream, "value", stream) or 0)
+
+
 def _torch_stream(device: torch.device, stream: int):
     """The stream a raw handle stands for (0 and 1: the null stream)."""
     if stream in (0, 1):
@@ -66,7 +70,8 @@ class _Workspace:
 
     def __init__(self, device: torch.device, stream: int, nbytes: int):
         self.idle_device = device if stream == _STREAM_PER_THREAD else None
-        with torch.cuda.stream(_torch_stream(device, 0 if self.idle_device else stream)):
+        self.stream = _torch_stream(device, 0 if self.idle_device else stream)
+        with torch.cuda.stream(self.stream):
             self.buf = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
         if self.idle_device:
             torch.cuda.synchronize(device)
@@ -82,7 +87,7 @@ def _workspace(device: torch.device, stream: int | None, nbytes: int) -> torch.T
         # memory of the graph's own, which its replays keep
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    stream = int(getattr(stream, "value", stream) or 0)
+    stream = _handle(stream)
     kept = getattr(_local, "workspaces", None)
     if kept is None:
         kept = _local.workspaces = OrderedDict()
@@ -95,14 +100,31 @@ def _workspace(device: torch.device, stream: int | None, nbytes: int) -> torch.T
     return ws.buf
 
 
-def _frames_u8(x, device=None) -> torch.Tensor:
+def _dense(x: torch.Tensor, stream: int | None, device=None) -> torch.Tensor:
+    """x in contiguous device memory. A copy is made on the stream that reads it and
+    is its memory: it is written after what the stream holds already, and what
+    takes the place of it next runs behind the kernels that read it."""
+    if x.is_cuda and x.is_contiguous():
+        return x
+    device = x.device if x.is_cuda else torch.device(device or "cuda")
+    if device.index is None:
+        device = torch.device(device.type, torch.cuda.current_device())
+    ws = _Workspace(device, _handle(stream), x.numel() * x.element_size())
+    out = ws.buf[:x.numel() * x.element_size()].view(x.dtype).view(x.shape)
+    with torch.cuda.stream(ws.stream):
+        out.copy_(x)
+    if ws.idle_device:
+        torch.cuda.synchronize(device)
+    out.workspace = ws
+    return out
+
+
+def _frames_u8(x, device=None, stream: int | None = None) -> torch.Tensor:
     if isinstance(x, np.ndarray):
         x = torch.from_numpy(np.ascontiguousarray(x))
     if x.dtype != torch.uint8:
         raise ValueError("frames must be uint8 gray images")
-    if not x.is_cuda:
-        x = x.to(device or "cuda")
-    return x.contiguous()
+    return _dense(x, stream, device)
 
 
 def _params(kw) -> dict:
@@ -118,7 +140,7 @@ def farneback_flows(frames, flows: torch.Tensor | None = None, stream: int | Non
                     **params) -> torch.Tensor:
     """Flow of every consecutive pair of a clip: frames uint8 [n, H, W] ->
     fp32 [n-1, H, W, 2] on the device, pair p = (frames[p], frames[p+1])."""
-    fr = _frames_u8(frames)
+    fr = _frames_u8(frames, stream=stream)
     if fr.dim() != 3:
         raise ValueError("frames must be [n, H, W]")
     n, H, W = fr.shape
@@ -149,7 +171,7 @@ def farneback_profile(frames, flows: torch.Tensor | None = None, stream: int | N
     -> (flows, [(kind name, pyramid level, ms), ...] in launch order), one entry for
     each kernel, level and iteration; the launches that a long clip's chunks of pairs
     take of it are summed."""
-    fr = _frames_u8(frames)
+    fr = _frames_u8(frames, stream=stream)
     n, H, W = fr.shape
     p = _params(params)
     lib = _lib.load()
@@ -180,8 +202,8 @@ def calc_optical_flow_farneback(prev, next, flow=None, pyr_scale=0.5, levels=3, 
     """cv2.calcOpticalFlowFarneback's argument order and meaning; prev/next
     uint8 [H, W] -> flow fp32 [H, W, 2] (dx, dy) on the device. A given
     ``flow`` tensor receives the result (flags must be 0: no initial flow)."""
-    a = _frames_u8(prev)
-    b = _frames_u8(next, a.device)
+    a = _frames_u8(prev, stream=stream)
+    b = _frames_u8(next, a.device, stream)
     if a.shape != b.shape or a.dim() != 2:
         raise ValueError("prev and next must be uint8 [H, W] of one size")
     H, W = a.shape
@@ -206,9 +228,9 @@ def change_rates(flows: torch.Tensor, grid_rows: int = 30, grid_cols: int = 52,
         flows = flows.unsqueeze(0)
     P, H, W, _ = flows.shape
     tiles = -(-(grid_rows * grid_cols) // tile_tokens)
-    fl = flows.contiguous()
-    cells = torch.empty(P, grid_rows, grid_cols, dtype=torch.float32, device=flows.device)
-    change = torch.empty(P, tiles, dtype=torch.float64, device=flows.device)
+    fl = _dense(flows, stream)
+    cells = torch.empty(P, grid_rows, grid_cols, dtype=torch.float32, device=fl.device)
+    change = torch.empty(P, tiles, dtype=torch.float64, device=fl.device)
     _check(_lib.load().kvp_motion_change_rates(_ptr(fl), P, W, H, grid_rows,
                                                grid_cols, tile_tokens, _ptr(cells), _ptr(change),
                                                stream), "kvp_motion_change_rates")

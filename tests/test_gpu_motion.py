@@ -437,3 +437,24 @@ def test_captured_flow_replays_between_eager_calls():
         eager = motion.farneback_flows((a, b)[1 - i % 2])
         torch.cuda.synchronize()
         assert torch.equal(out, want[i % 2]) and torch.equal(eager, want[1 - i % 2]), i
+
+
+@pytest.mark.parametrize("per_thread", [False, True])
+def test_copied_inputs_outlive_the_call_on_its_stream(per_thread):
+    """Strided frames and flows are copied for the call; the copies' memory must not be
+    handed to another stream's tensors while the call's kernels read it."""
+    clip = torch.from_numpy(workloads.synthetic_clip(12, 480, 832, seed=5)).to(DEV)
+    want = motion.farneback_flows(clip)
+    rates = motion.change_rates(want)
+    wide = torch.stack([clip, clip], dim=-1)[..., 0]
+    both = torch.stack([want, want], dim=-1)[..., 0]
+    out = torch.full_like(want, float("nan"))
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    stream = 2 if per_thread else side.cuda_stream
+    motion.farneback_flows(wide, out, stream=stream)
+    cells, change = motion.change_rates(both, stream=stream)
+    junk = [torch.full((12, 480, 832), 255, dtype=torch.uint8, device=DEV) for _ in range(8)]
+    junk += [torch.full_like(want, float("nan")) for _ in range(4)]
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(cells, rates[0]) and torch.equal(change, rates[1])

@@ -44,8 +44,12 @@ def test_csv_round_trip(tmp_path):
 def on_host(monkeypatch):
     """motion._workspace with host tensors in place of device memory."""
     class Host:
+        stream = idle_device = None
+        made = []
+
         def __init__(self, device, stream, nbytes):
             self.buf = torch.empty(nbytes, dtype=torch.uint8)
+            self.made.append((device, stream, nbytes))
 
     monkeypatch.setattr(motion, "_Workspace", Host)
     monkeypatch.setattr(motion, "_local", threading.local())
@@ -81,3 +85,15 @@ def test_a_thread_keeps_a_bounded_number_of_workspaces(on_host):
     motion._workspace(on_host, 0x10000, 1)
     assert len(kept) == motion._MAX_WORKSPACES and (0, 0x200) not in kept
     assert motion._workspace(on_host, 0x200, 1) is not second
+
+
+def test_copied_frames_belong_to_the_stream_that_reads_them(on_host, monkeypatch):
+    """Host frames and strided ones are copied into memory of the call's stream."""
+    made = motion._Workspace.made
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    frames = np.random.default_rng(4).integers(0, 256, (2, 12, 10), dtype=np.uint8)
+    got = motion._frames_u8(frames[:, :, ::2], stream=0x1000)
+    assert made == [(on_host, 0x1000, 120)] and np.array_equal(got.numpy(), frames[:, :, ::2])
+    flows = torch.arange(48, dtype=torch.float32).view(4, 3, 4)[:, :, :2]
+    got = motion._dense(flows, None, on_host)
+    assert made[1] == (on_host, 0, 4 * 24) and torch.equal(got, flows) and got.is_contiguous()
