@@ -41,6 +41,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "kvp_internal.h"
 
@@ -639,6 +640,22 @@ int choose_tile(long rows, int features) {
     return jr;
 }
 
+// Shapes the tiled kernels take: whole 128-byte chunks of K, whole feature tiles,
+// operand tiles addressed with 32-bit offsets.
+bool tileable(int in_dtype, int K, int N, int tile_n) {
+    const long kbytes = (long)K * (in_dtype == 0 ? 4 : 2);
+    return kbytes % kPRowBytes == 0 && N % tile_n == 0 && kbytes * kWTileN <= 0x7fffffffL;
+}
+
+// Tiled kernel of a launch over features in all groups, as kvp_linear_kernel
+// reports it: 2 = 128 x 128, 3 = 256 x 256, 4 = 256 features x 320 tokens.
+int tiled_kernel(int in_dtype, long rows, int K, int features) {
+    if (in_dtype == 0) return 2;
+    const int jr = choose_tile(rows, features);
+    // (a tile's tokens are addressed with 32-bit offsets)
+    return jr == 0 || 128L * jr * K > 0x7fffffffL ? 2 : jr - 1;
+}
+
 template <typename InT, typename OutT, bool kAcc>
 void launch_small(const ProjArgs& a, hipStream_t st) {
     const int grid = a.n_tiles * a.r_tiles;
@@ -795,15 +812,16 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GenericArgs a) {
 // 64 x 64 tiles of gemm_generic_kernel pad K to 32 and stage both operands
 // through LDS for one chunk of work. 12480 rows x 16 -> 1536 features:
 // 51 -> 32 us (2.4 TB/s written). 8 rows per wave 32.6 us, 32 rows 38.7.
+// short_inner says where it is used.
 constexpr int kThinRows = 16;
 constexpr int kThinCols = 256;
 
-template <int kK>
+template <int kK, bool kAcc>
 __global__ __launch_bounds__(256) void gemm_thin_kernel(const float* __restrict__ X,
                                                          const float* __restrict__ W,
                                                          const float* __restrict__ bias,
                                                          float* __restrict__ Y, long rows, int N,
-                                                         int n_tiles, int accumulate) {
+                                                         int n_tiles) {
     static_assert(kK % 4 == 0 && kK <= 16, "4 kK weights per lane");
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     constexpr int kPitch = kThinCols + 4;  // 16 columns x 4 k's quads: 64 banks
@@ -825,8 +843,10 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const float* __restrict_
     float4 w[kK];
 #pragma unroll
     for (int k = 0; k < kK; ++k) w[k] = *reinterpret_cast<const float4*>(ws + k * kPitch + c);
-    const float4 b = bias ? *reinterpret_cast<const float4*>(bias + n)
-                          : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 b = bias ? *reinterpret_cast<const float4*>(bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+    // wait for the bias here: its first use is in the loop, where the wait for it
+    // would be one for the store of the row before, too
+    asm volatile("" : "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w));
     const long end = min(r0 + kThinRows, rows);
     Y += n;
 #pragma unroll 4
@@ -842,12 +862,27 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const float* __restrict_
         }
         v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
         float4* y = reinterpret_cast<float4*>(Y + r * N);
-        if (accumulate) {
+        if constexpr (kAcc) {
             const float4 o = *y;
             v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
         }
         *y = v;
     }
+}
+
+// Whether the kernel above takes an fp32 layer (16-byte aligned operands). Its
+// waves write rows one by one: stores of less than 256 bytes (512 for 16 inputs)
+// hold them up, also in a last column block of few features, which only the work
+// of many other blocks hides; few rows leave no work to gain from. Any-shape
+// kernel -> this one, us:
+// 12480 rows, 16 -> 1536 36.3 -> 19.2, 16 -> 256 11.2 -> 7.3, 16 -> 64 6.5 -> 6.4
+// (60000 rows: 1.2 times as long), 16 -> 4 5.2 -> 11.3; 16 -> 260 at 1560 rows
+// 6.3 -> 10.9, at 20000 0.80 of the time; 8 -> 64 at 1560 rows 6.1 -> 5.2; 4 -> 4
+// at 12480 rows 5.2 -> 5.2, at 200000 17.3 -> 11.5.
+bool short_inner(long rows, int K, int N) {
+    if (K > 16 || K % 4 || N % 4 || rows < 64) return false;
+    const int last = (N - 1) % kThinCols + 1;  // features of the last column block
+    return K == 4 || last >= (K < 16 ? 64 : 128) || (long)(N / kThinCols) * rows >= 16384;
 }
 
 template <typename InT, typename OutT, bool kAcc>
@@ -887,9 +922,7 @@ int launch_gemm_generic(int in_dtype, int out_dtype, const void* x, const void* 
     a.rows = rows;
     a.K = K;
     a.N = N;
-    // weights that fit a lane's registers, in whole 16-byte groups of weights,
-    // bias and output (both sides measured: 32 and 51 us, see the kernel)
-    const bool thin = in_dtype == 0 && K <= 16 && K % 4 == 0 && N % 4 == 0 &&
+    const bool thin = in_dtype == 0 && short_inner(rows, K, N) &&
                       ((uintptr_t)w | (uintptr_t)bias | (uintptr_t)y) % 16 == 0;
     const int cols = thin ? kThinCols : kGTile;
     const int tile_rows = thin ? 4 * kThinRows : kGTile;
@@ -906,14 +939,21 @@ int launch_gemm_generic(int in_dtype, int out_dtype, const void* x, const void* 
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st,
                                static_cast<const float*>(x), static_cast<const float*>(w), bias,
-                               static_cast<float*>(y), rows, N, a.n_tiles, (int)accumulate);
+                               static_cast<float*>(y), rows, N, a.n_tiles);
         };
-        switch (K) {
-            case 4: go(gemm_thin_kernel<4>); break;
-            case 8: go(gemm_thin_kernel<8>); break;
-            case 12: go(gemm_thin_kernel<12>); break;
-            default: go(gemm_thin_kernel<16>);
-        }
+        auto pick = [&](auto acc) {
+            constexpr bool kAcc = decltype(acc)::value;
+            switch (K) {
+                case 4: go(gemm_thin_kernel<4, kAcc>); break;
+                case 8: go(gemm_thin_kernel<8, kAcc>); break;
+                case 12: go(gemm_thin_kernel<12, kAcc>); break;
+                default: go(gemm_thin_kernel<16, kAcc>);
+            }
+        };
+        if (accumulate)
+            pick(std::true_type{});
+        else
+            pick(std::false_type{});
     } else if (in_dtype == 0) {
         if (accumulate)
             launch_generic<float, float, true>(a, grid, st);
@@ -949,8 +989,7 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
         set_error("proj_gemm: fp32 operands need tile_n 128 and fp32 output");
         return 1;
     }
-    const long kbytes = (long)K * (in_dtype == 0 ? 4 : 2);
-    if (kbytes % kPRowBytes || Ng % tile_n || kbytes * kWTileN > 0x7fffffffL) {
+    if (!tileable(in_dtype, K, Ng, tile_n)) {
         set_error("proj_gemm: shape K=%d N=%d not supported (K %% %d, N %% %d)", K, Ng,
                   in_dtype == 0 ? kPChunkK / 2 : kPChunkK, tile_n);
         return 2;
@@ -999,12 +1038,11 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
         else
             launch_small<float, float, false>(a, st);
     } else {
-        int jr = tile_n == 256 ? 4 : choose_tile(rows, groups * Ng);
-        // (a tile's tokens are addressed with 32-bit offsets)
-        if (64 * jr * kbytes > 0x7fffffffL) jr = 0;
-        if (jr == 5)
+        const int kernel =
+            tile_n == 256 ? 3 : tiled_kernel(in_dtype, rows, K, groups * Ng);
+        if (kernel == 4)
             launch_wide<5>(a, out_dtype, accumulate, st);
-        else if (jr == 4)
+        else if (kernel == 3)
             launch_wide<4>(a, out_dtype, accumulate, st);
         else if (out_dtype == 1)
             launch_small<__bf16, __bf16, false>(a, st);
@@ -1022,6 +1060,19 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
 }
 
 }  // namespace kvp
+
+extern "C" int kvp_linear_kernel(int in_dtype, int out_dtype, long rows, int in_features,
+                                 int out_features, int groups, int accumulate) {
+    using namespace kvp;
+    const int K = in_features, N = out_features;
+    const bool types = (in_dtype == 1 && (out_dtype == 0 || out_dtype == 1)) ||
+                       (in_dtype == 0 && out_dtype == 0);
+    if (!types || (accumulate && out_dtype != 0) || rows <= 0 || K <= 0 || N <= 0 || groups < 1 ||
+        groups > 3)
+        return -1;
+    if (tileable(in_dtype, K, N, kPSmall)) return tiled_kernel(in_dtype, rows, K, groups * N);
+    return in_dtype == 0 && short_inner(rows, K, N) ? 1 : 0;
+}
 
 extern "C" int kvp_proj_gemm(const void* x, const void* w, const float* bias, void* out0,
                              void* out1, void* out2, int groups, long rows, int K, int N,

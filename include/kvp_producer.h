@@ -41,6 +41,14 @@ int kvp_linear(int in_dtype, int out_dtype, const void* x, const void* w,
                const float* bias, void* y, long rows, int in_features,
                int out_features, int accumulate, void* stream);
 
+/* The kernel kvp_linear (groups 1) or the grouped projection (up to 3 groups of
+ * out features) runs for operands that are 16-byte aligned, by the rules on
+ * sizes alone: 0 any-shape, 1 short inner dimension, tiles of 2 = 128 features x
+ * 128 tokens, 3 = 256 x 256, 4 = 256 x 320; -1 for what they refuse. For tests
+ * and measurement; needs no GPU. */
+int kvp_linear_kernel(int in_dtype, int out_dtype, long rows, int in_features,
+                      int out_features, int groups, int accumulate);
+
 /* Grouped bf16 projection on this library's gfx950 MFMA kernel: for
  * g < groups (1..3), out_g[r, n] = x[r, :] . w[g*N + n, :] + bias[g*N + n]
  * (+ out_g[r, n] when accumulate != 0). x [rows, K] and w [groups*N, K]

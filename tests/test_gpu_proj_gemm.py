@@ -116,6 +116,18 @@ def test_fp32_linear_short_inner(rows, K, N, acc, bias):
     _check_fp32_linear(rows, K, N, acc, bias)
 
 
+# the same where the register kernel is the one that runs: rows around a wave's
+# 16 and a block's 64, column blocks that end after 64, 128, 252 and 44 features
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N,acc,bias", [
+    (64, 4, 4, False, True), (65, 8, 64, True, True), (79, 12, 252, False, False),
+    (130, 16, 128, True, False), (81, 16, 512, False, True), (16385, 8, 300, True, True),
+])
+def test_fp32_linear_short_inner_kernel(lib, rows, K, N, acc, bias):
+    assert lib.kvp_linear_kernel(0, 0, rows, K, N, 1, int(acc)) == 1
+    _check_fp32_linear(rows, K, N, acc, bias)
+
+
 def _check_fp32_linear(rows, K, N, acc, bias):
     print(f"fp32 linear rows={rows} K={K} N={N} acc={acc}", flush=True)
     rng = np.random.default_rng(rows + K + N)
