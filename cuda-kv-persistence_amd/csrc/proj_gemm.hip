@@ -615,14 +615,22 @@ void launch_wide(const ProjArgs& a, int out_dtype, bool accumulate, hipStream_t 
 
 // Tile of a bf16 launch: 0 = 128 x 128, else JR of the wide form (4: 256 x 256,
 // 5: 256 x 320). Each form's time is its rounds over the chip times the measured
-// time of a round (K = 1536; every term scales with K alike): 128 x 128 fills
-// 512 slots in 29 us, and its tiles even out beyond the first round; 256 x 256
-// takes 43.6 us a round of 256, 256 x 320 51 us. All three add the same terms
-// in the same order: results are equal bit for bit. Measured (us; 128 x 128,
-// 256 x 256, 256 x 320): 12480 tokens x 3 x 1536 features 205, 175, 153; x 1536
-// accumulating 85, 95, 69; 8000 x 3 x 1664 135, 132, 114; x 1664 65, 55, 62;
-// 5365 x 3 x 1152 52, 59, 42; 1560 x 3 x 1536 27, 38, 41.
-int choose_tile(long rows, int features) {
+// time of a round (K = 1536): 128 x 128 fills 512 slots in 29 us, and its tiles
+// even out beyond the first round; 256 x 256 takes 43.6 us a round of 256, 256 x
+// 320 51 us. With few chunks of K a launch is bound by its outputs, which the
+// 128 x 128 form writes (and, accumulating, whose residual it reads) under its
+// other workgroup's MFMAs; the wide forms' one workgroup a CU does not. So these
+// take K from 256, accumulating from 768. All three add the same terms in the
+// same order: results are equal bit for bit. Measured, the card kept busy (us;
+// 128 x 128, 256 x 256, 256 x 320):
+//   K = 1536: 12480 tokens x 4608 features 174, 169, 149; x 1536 accumulating 78,
+//   93, 66; 9000 x 3072 91, 84, 92; 3120 x 4608 49, 44, 47; 1560 x 4608 27, 38, 41
+//   12480 x 3072, K = 512: 53, 53, 44; K = 256: 34, 36, 30; 12480 x 4608, K = 192:
+//   41, 44, 41; K = 128: 33, 37, 35; 9000 x 6144, K = 128: 32, 38, 35
+//   12480 x 3072 accumulating, K = 1024: 105, 114, 100; K = 512: 72, 80, 72;
+//   K = 256: 56, 67, 58; 28000 x 3072, K = 512: 180, 198, 201
+int choose_tile(long rows, int K, int features, bool accumulate) {
+    if (K < (accumulate ? 768 : 256)) return 0;
     const double small_tiles =
         (double)((rows + kPSmall - 1) / kPSmall) * ((features + kPSmall - 1) / kPSmall);
     double best = 29.0 * (small_tiles > 2 * kPCus ? small_tiles / (2 * kPCus) : 1.0);
@@ -649,9 +657,9 @@ bool tileable(int in_dtype, int K, int N, int tile_n) {
 
 // Tiled kernel of a launch over features in all groups, as kvp_linear_kernel
 // reports it: 2 = 128 x 128, 3 = 256 x 256, 4 = 256 features x 320 tokens.
-int tiled_kernel(int in_dtype, long rows, int K, int features) {
+int tiled_kernel(int in_dtype, long rows, int K, int features, bool accumulate) {
     if (in_dtype == 0) return 2;
-    const int jr = choose_tile(rows, features);
+    const int jr = choose_tile(rows, K, features, accumulate);
     // (a tile's tokens are addressed with 32-bit offsets)
     return jr == 0 || 128L * jr * K > 0x7fffffffL ? 2 : jr - 1;
 }
@@ -1040,7 +1048,7 @@ int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bi
             launch_small<float, float, false>(a, st);
     } else {
         const int kernel =
-            tile_n == 256 ? 3 : tiled_kernel(in_dtype, rows, K, groups * Ng);
+            tile_n == 256 ? 3 : tiled_kernel(in_dtype, rows, K, groups * Ng, accumulate);
         if (kernel == 4)
             launch_wide<5>(a, out_dtype, accumulate, st);
         else if (kernel == 3)
@@ -1071,7 +1079,8 @@ extern "C" int kvp_linear_kernel(int in_dtype, int out_dtype, long rows, int in_
     if (!types || (accumulate && out_dtype != 0) || rows <= 0 || K <= 0 || N <= 0 || groups < 1 ||
         groups > 3)
         return -1;
-    if (tileable(in_dtype, K, N, kPSmall)) return tiled_kernel(in_dtype, rows, K, groups * N);
+    if (tileable(in_dtype, K, N, kPSmall))
+        return tiled_kernel(in_dtype, rows, K, groups * N, accumulate != 0);
     return in_dtype == 0 && short_inner(rows, K, N) ? 1 : 0;
 }
 

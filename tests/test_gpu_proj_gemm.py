@@ -180,3 +180,39 @@ def test_fp32_qkv_project_is_three_linears(rows, heads):
 ])
 def test_wide_tiles_match_oracle(rows, K, N, groups, tile_n, out_dt, acc, bias):
     test_proj_gemm_matches_oracle(rows, K, N, groups, tile_n, out_dt, acc, bias)
+
+
+# the same where a launch picks the wide tiles itself (K from 256, from 768 when it
+# accumulates), with features past the last group and a wave's accumulators there
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N,groups,out_dt,acc,kernel", [
+    (12473, 256, 1408, 3, 1, False, 4), (12473, 256, 384, 3, 0, False, 3),
+    (12473, 768, 1408, 1, 0, True, 4), (3117, 256, 1408, 3, 1, False, 3),
+    (3117, 768, 4480, 1, 0, True, 3),
+])
+def test_chosen_wide_tiles_match_oracle(lib, rows, K, N, groups, out_dt, acc, kernel):
+    assert lib.kvp_linear_kernel(1, out_dt, rows, K, N, groups, int(acc)) == kernel
+    test_proj_gemm_matches_oracle(rows, K, N, groups, 128, out_dt, acc, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out_dt,acc", [(1, False), (0, False), (0, True)])
+def test_all_tiles_give_the_same_bits(lib, out_dt, acc):
+    """The same rows through 256 x 320, 256 x 256 and 128 x 128 tiles."""
+    rows, K, N, few = 12473, 768, 1536, 1500
+    print(f"tiles bitwise out={out_dt} acc={acc}", flush=True)
+    kernels = [lib.kvp_linear_kernel(1, out_dt, r, K, N, 1, int(acc)) for r in (rows, few)]
+    assert kernels == [4, 2]
+    g = torch.Generator(device=DEV).manual_seed(out_dt + 2 * acc)
+    x = torch.randn(rows, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (0.02 * torch.randn(N, K, generator=g, device=DEV)).to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device=DEV)
+    odt = torch.bfloat16 if out_dt else torch.float32
+    y0 = torch.randn(rows, N, generator=g, device=DEV).to(odt)
+    outs = []
+    for n, tile_n in ((rows, 128), (rows, 256), (few, 128)):
+        y = y0.clone()
+        kb.proj_gemm(x[:n], w, b, [y[:n]], accumulate=acc, tile_n=tile_n)
+        outs.append(y)
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0][:few], outs[2][:few]) and torch.equal(outs[2][few:], y0[few:])

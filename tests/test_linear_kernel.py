@@ -29,6 +29,26 @@ def test_short_inner_fp32(lib, rows, K, N, want):
     assert _kernel(lib, BF16, rows, K, N) == ANY
 
 
+@pytest.mark.parametrize("rows,K,N,groups,out_dtype,acc,want", [
+    (12480, 1536, 1536, 3, BF16, False, 4), (12480, 1536, 1536, 1, FP32, True, 4),
+    (3120, 1536, 1536, 3, BF16, False, 3), (1560, 1536, 1536, 3, BF16, False, 2),
+    # few chunks of K
+    (12480, 128, 4608, 1, BF16, False, 2), (12480, 192, 1536, 3, BF16, False, 2),
+    (12480, 256, 1536, 3, BF16, False, 4), (12480, 704, 3072, 1, FP32, True, 2),
+    (12480, 768, 3072, 1, FP32, True, 4), (12480, 704, 3072, 1, FP32, False, 4),
+    # not tiled: K not a multiple of 64, N of 128
+    (12480, 1568, 1536, 1, BF16, False, ANY), (12480, 1536, 1500, 1, BF16, False, ANY),
+])
+def test_bf16_tiles(lib, rows, K, N, groups, out_dtype, acc, want):
+    assert _kernel(lib, BF16, rows, K, N, groups, out_dtype, acc) == want
+
+
+def test_fp32_tiles_are_128_by_128(lib):
+    assert _kernel(lib, FP32, 12480, 1536, 1536, 3) == 2
+    assert _kernel(lib, FP32, 1, 32, 128, acc=True) == 2
+    assert _kernel(lib, FP32, 12480, 48, 1536) == ANY
+
+
 @pytest.mark.parametrize("args", [
     (FP32, BF16, 8, 64, 128, 1, 0), (2, 0, 8, 64, 128, 1, 0), (BF16, BF16, 8, 64, 128, 1, 1),
     (FP32, FP32, 0, 64, 128, 1, 0), (FP32, FP32, 8, 0, 128, 1, 0), (FP32, FP32, 8, 64, 128, 4, 0),
