@@ -74,7 +74,8 @@ constexpr int kPbRows = 32;                         // source rows under a block
 constexpr size_t kPbLdsBytes = 64 << 10;            // rows are cut to what fits this
 constexpr int kPyrLevels = 9;                       // 8192 px down to 32 px at scale 0.5
 constexpr int kPyrTaps = 512;
-constexpr long kChunkPixels = 17L * 832 * 480;      // pixels x pairs of a chunk
+constexpr long kStepChunkPixels = 17L * 832 * 480;  // pixels x pairs of a chunk: window 15,
+constexpr long kChunkPixels = 32 * kStepChunkPixels;  // and any other
 constexpr int kBfBatch = 4;       // box filter: rows parked in LDS at a time
 constexpr int kBfRun = 2;         // box filter: output columns per sliding run
 constexpr int kBfTargetGroups = 2048;
@@ -1084,23 +1085,32 @@ void flow_strips(int w, int h, int n, FlowArgs& a) {
     }
 }
 
-// Pairs of a level taken at a time, in equal shares: their expansions and two
-// flow buffers (36 B per pixel) then stay in the 256 MiB Infinity Cache from one
-// iteration to the next. A 50-frame 832x480 clip takes 1,488 us in 3 chunks of 17
-// pairs, 1,580 in 5 of 10 and 1,551 in 2 of 25.
-int chunk_pairs(long pixels, int pairs) {
-    const long cap = std::max<long>(1, kChunkPixels / pixels);
+// Pairs of a level taken at a time, in equal shares.
+//
+// flow_step_kernel (`step`): 17 x 832 x 480 pixels, whose expansions and two flow
+// buffers (36 B per pixel) stay in the 256 MiB Infinity Cache from one iteration to
+// the next. A chunk's last round of strips costs what that gains, or more on large
+// frames: in chunks and in one launch, 50 frames of 832x480 1511 and 1504 us, 100 of
+// 416x240 760 and 809, 100 of 832x480 3003 and 3063, 30 of 1920x1080 4875 and 4757,
+// 12 of 3840x2160 7930 and 7080.
+//
+// Other windows: all pairs, but for clips whose full-size expansions and matrices
+// (40 B a pixel and pair) would take more than 8.7 GB. Their matrices do not stay in
+// the cache, and in short launches their blocks' rows are few for the window (their
+// halo). 30 frames of 1920x1080 in chunks of 17 x 832 x 480 pixels and in one launch:
+// window 9 6890 and 6259 us, 49 11753 and 9779; 20 of 832x480, window 33, 1492 and 1343.
+int chunk_pairs(long pixels, int pairs, bool step) {
+    const long cap = std::max<long>(1, (step ? kStepChunkPixels : kChunkPixels) / pixels);
     const long chunks = (pairs + cap - 1) / cap;
     return (int)((pairs + chunks - 1) / chunks);
 }
 
-// Workspace: the reduced levels' images and expansions for all frames, the
-// full-size level's expansions for one chunk of pairs, two flow buffers of the
+// Workspace for any window: the reduced levels' images and expansions for all
+// frames, the full-size level's expansions for one chunk of pairs, two flow buffers of the
 // largest reduced level, and a region that holds either the matrices of a chunk
 // or the second flow buffer of its iterations, whichever the window size needs.
 struct Layout {
     std::vector<size_t> img, R;  // per plan entry
-    std::vector<int> chunk;
     size_t fa, fb, M, total;
 };
 
@@ -1116,8 +1126,7 @@ Layout layout(int nf, int W, int H, const std::vector<Level>& plan) {
     };
     for (const Level& l : plan) {
         const size_t P = (size_t)l.w * l.h;
-        const int chunk = chunk_pairs((long)P, pairs);
-        L.chunk.push_back(chunk);
+        const int chunk = chunk_pairs((long)P, pairs, false);  // the larger of the two
         L.img.push_back(l.k > 0 ? take(nf * P) : 0);
         L.R.push_back(take((l.k > 0 ? (size_t)nf : chunk + 1) * 5 * P));
         if (l.k > 0) P1 = std::max(P1, P);
@@ -1254,6 +1263,9 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
     float2* fbuf[2] = {(float2*)(ws + L.fa), (float2*)(ws + L.fb)};
     const int pairs = nf - 1;
     const int m = winsize / 2;
+    const bool step = m == kFsHalf && iterations > 0;  // flow_step_kernel
+    std::vector<int> chunk;  // per plan entry
+    for (const Level& l : plan) chunk.push_back(chunk_pairs((long)l.w * l.h, pairs, step));
     const double box_scale = 1.0 / ((double)winsize * winsize);
 
     auto mark = [&](int kind, int lv, int iteration = 0) {
@@ -1317,7 +1329,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
                     v.img = -1;
                 }
                 v.R = (long)(L.R[l0] / sizeof(float));
-                v.slots = l.k > 0 ? nf : L.chunk[l0] + 1;
+                v.slots = l.k > 0 ? nf : chunk[l0] + 1;
                 v.tiles_x = (l.w + kPeTileW - 1) / kPeTileW;
                 v.first_block = poly_blocks;
                 poly_blocks += v.tiles_x * ((l.h + kPeTileH - 1) / kPeTileH);
@@ -1339,7 +1351,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
     // The full-size level (the last of the plan) is expanded chunk by chunk,
     // or with the others where one chunk holds every pair.
     const size_t last = plan.size() - 1;
-    const bool whole = L.chunk[last] >= pairs;
+    const bool whole = chunk[last] >= pairs;
     if (pyramid(0, whole ? last + 1 : last, 0, nf)) return 1;
 
     // Iterations of plan level li for pairs [p0, p0 + n).
@@ -1352,7 +1364,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
         FlowArgs a = {};
         a.R = (const float*)(ws + L.R[li]);
         a.first_pair = p0;
-        a.slots = l.k > 0 ? nf : L.chunk[li] + 1;
+        a.slots = l.k > 0 ? nf : chunk[li] + 1;
         a.w = l.w;
         a.h = l.h;
         a.box_scale = box_scale;
@@ -1365,7 +1377,7 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
             a.cy_scale = 1.0 / ((double)l.h / a.ch);
         }
         const dim3 pix((unsigned)((P + 255) / 256), n);
-        if (m == kFsHalf && iterations > 0) {
+        if (step) {
             // iteration i writes what i + 1 reads: two buffers in turn, the
             // last one fl
             float2* other = (float2*)M;
@@ -1417,8 +1429,8 @@ int farneback_impl(const uint8_t* frames, long frame_stride, int nf, int W, int 
     };
 
     for (size_t li = 0; li <= last; ++li) {
-        for (int p0 = 0; p0 < pairs; p0 += L.chunk[li]) {
-            const int n = std::min(L.chunk[li], pairs - p0);
+        for (int p0 = 0; p0 < pairs; p0 += chunk[li]) {
+            const int n = std::min(chunk[li], pairs - p0);
             // a later chunk's first frame is the last of the chunk before it
             const int f0 = p0 == 0 ? 0 : p0 + 1;
             if (li == last && !whole && pyramid(last, last + 1, f0, p0 + n + 1 - f0)) return 1;

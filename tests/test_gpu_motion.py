@@ -356,18 +356,37 @@ def test_pyramid_and_strip_edges_match_oracle(H, W, params):
     _flow_ok(got, fb.calc_optical_flow_farneback(clip[0], clip[1], **params), f"{H}x{W} {params}")
 
 
-def _steps(frames, H, W, **params):
-    clip = torch.from_numpy(workloads.synthetic_clip(frames, H, W, seed=frames)).to(DEV)
+def _steps(clip, **params):
     flows, steps = motion.farneback_profile(clip, **params)
     assert torch.equal(flows, motion.farneback_flows(clip, **params))
     assert all(ms > 0 for _, _, ms in steps)
     return [(kind, level) for kind, level, _ in steps]
 
 
-@pytest.mark.parametrize("params", [{}, dict(winsize=9)])
-def test_profile_entries_do_not_grow_with_the_clip(params):
-    """20 and 60 frames of 832x480 take 2 and 4 chunks of the full-size level's pairs."""
-    assert _steps(20, 480, 832, **params) == _steps(60, 480, 832, **params)
+def _rolled_clip(frames, H, W):
+    """A smooth random image that moves by a pixel or two from frame to frame, made on the device."""
+    g = torch.Generator(device=DEV).manual_seed(H + W)
+    image = torch.nn.functional.avg_pool2d(torch.randn(1, 1, H + 8, W + 8, generator=g, device=DEV),
+                                           9, 1)[0, 0]
+    image = (128 + 300 * image).clamp(0, 255).to(torch.uint8)
+    return torch.stack([torch.roll(image, (f, 2 * f), (0, 1)) for f in range(frames)])
+
+
+@pytest.mark.parametrize("frames,H,W,params", [
+    (20, 480, 832, {}), (14, 4096, 4096, dict(winsize=9))])
+def test_profile_entries_do_not_grow_with_the_clip(frames, H, W, params):
+    """Three times the frames take 2 and 4 chunks of the full-size level's pairs."""
+    clip = _rolled_clip(3 * frames, H, W)
+    assert _steps(clip[:frames], **params) == _steps(clip, **params)
+
+
+def test_other_windows_in_chunks_equal_their_pairs_bitwise():
+    """13 pairs of 4096x4096 are two chunks for a window that runs in several launches."""
+    clip = _rolled_clip(14, 4096, 4096)
+    flows = motion.farneback_flows(clip, winsize=9)
+    for p in (0, 6, 7, 12):
+        pair = motion.calc_optical_flow_farneback(clip[p], clip[p + 1], winsize=9)
+        assert torch.equal(flows[p], pair), p
 
 
 def test_profile_levels():
@@ -377,8 +396,9 @@ def test_profile_levels():
     flow = lambda lv, first: [(first, lv)] * (first is not None) + [(motion.KINDS[4], lv)] * 3
     blur, expand, init = motion.KINDS[1:4]
     coarse = flow(3, None) + flow(2, init) + flow(1, init)
-    assert _steps(2, 480, 832) == [(blur, 1), (expand, 0)] + coarse + flow(0, init)
-    assert _steps(20, 480, 832) == [(blur, 1), (expand, 1)] + coarse + [(expand, 0)] + flow(0, init)
+    clip = _rolled_clip(20, 480, 832)
+    assert _steps(clip[:2]) == [(blur, 1), (expand, 0)] + coarse + flow(0, init)
+    assert _steps(clip) == [(blur, 1), (expand, 1)] + coarse + [(expand, 0)] + flow(0, init)
 
 
 def test_calls_overlapping_on_streams_and_threads_equal_serial_ones():
