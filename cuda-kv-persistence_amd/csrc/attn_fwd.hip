@@ -375,6 +375,10 @@ __device__ __forceinline__ u32x2 lds_tr16(unsigned addr) {
     return r;
 }
 
+__device__ __forceinline__ void lgkm_wait2(u32x4& a, u32x4& b) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b)::"memory");
+}
+
 // Waits for all but the two most recent LDS reads (LDS reads complete in
 // issue order and no scalar-memory load is issued in the compute phase).
 __device__ __forceinline__ void lgkm_wait2_keep2(u32x4& a, u32x4& b) {
@@ -841,15 +845,24 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     // the map 689 -> 648 us. Waves of 64 queries, one per SIMD, on the same
     // schedule: 16.3 ms and 153 us.
     // The values and the order in which they are added to O are those of the
-    // product taken in the tile's own step. The first step's pending product
-    // is 0 x 0.
+    // product taken in the tile's own step. The first step has no product
+    // pending and no running max to exponentiate against; it is a step of its
+    // own (kFirst) that leaves both out: key ranges of one tile 5.3 -> 4.5 us, 50
+    // frames of 900 tokens within themselves 295 -> 288. But without a map, walks
+    // of more than kShortWalk tiles gain less than their workgroups lose by
+    // starting in step (8 frames of 1560 tokens 126.4 -> 128.4): there the first
+    // step's pending product is 0 x 0.
+    constexpr int kShortWalk = 16;
+    const bool first_apart = kMap || ntiles <= kShortWalk;
     u32x4 pd[4];
+    if (!first_apart) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) pd[g] = u32x4{0u, 0u, 0u, 0u};
+        for (int g = 0; g < 4; ++g) pd[g] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int i = 0; i < kBf16TileBytes / 16 / kThreads; ++i)
-        *reinterpret_cast<u32x4*>(v_lds + 2 * kBf16TileBytes + 16 * (tid + kThreads * i)) =
-            u32x4{0u, 0u, 0u, 0u};
+        for (int i = 0; i < kBf16TileBytes / 16 / kThreads; ++i)
+            *reinterpret_cast<u32x4*>(v_lds + 2 * kBf16TileBytes + 16 * (tid + kThreads * i)) =
+                u32x4{0u, 0u, 0u, 0u};
+    }
     // V^T fragment j = 4 g + nb (k-step g of 16 keys, 32-column block nb): two
     // transposing reads, kAhead fragments ahead of its MFMA (2, 4, 6: within
     // 1 % of each other)
@@ -882,8 +895,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) vad[nb] = (unsigned)(uintptr_t)v_tile + vofs_nb[nb];
     };
-    auto compute_tile = [&](int t, const unsigned char* ks_lds, const unsigned char* v_prev,
-                            auto&& between, auto&& after) {
+    auto compute_tile = [&](auto first, int t, const unsigned char* ks_lds,
+                            const unsigned char* v_prev, auto&& between, auto&& after) {
+        constexpr bool kFirst = decltype(first)::value;
         const unsigned kbase = (unsigned)(uintptr_t)ks_lds + (unsigned)(lq * 256);
         unsigned vad[4];
         v_addr(v_prev, vad);
@@ -905,15 +919,20 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
         for (int ks = 0; ks < 8; ++ks) {
             const int cur = ks % 3;
             // behind them: the next K fragments, then V fragment 0
-            lgkm_wait2_keep2(ka[cur], kb[cur]);
+            if (kFirst && ks == 7)
+                lgkm_wait2(ka[cur], kb[cur]);
+            else
+                lgkm_wait2_keep2(ka[cur], kb[cur]);
             if (ks + 2 < 8) {
                 const int nx = (ks + 2) % 3;
                 const unsigned ad = kbase + ((((unsigned)(2 * (ks + 2) + hh)) ^ kswz) << 4);
                 ka[nx] = lds_b128<0>(ad);
                 kb[nx] = lds_b128<32 * 256>(ad);
             }
-            if (ks == 6) read_vd(std::integral_constant<int, 0>{}, vad);
-            if (ks == 7) read_vd(std::integral_constant<int, 1>{}, vad);
+            if constexpr (!kFirst) {
+                if (ks == 6) read_vd(std::integral_constant<int, 0>{}, vad);
+                if (ks == 7) read_vd(std::integral_constant<int, 1>{}, vad);
+            }
             s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ka[cur]),
                                                          qf[ks], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kb[cur]),
@@ -951,7 +970,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             pd[e / 4][e % 4] = __builtin_bit_cast(unsigned, w);
         };
         constexpr int kPack = 5;
-        static_for<16 + kPack>([&](auto mc) __attribute__((always_inline)) {
+        static_for<kFirst ? 0 : 16 + kPack>([&](auto mc) __attribute__((always_inline)) {
             constexpr int m = decltype(mc)::value;
             if constexpr (m < 16) {
                 pv_step(mc);
@@ -973,7 +992,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             if constexpr (m < 16) __builtin_amdgcn_sched_barrier(0);
         });
         float tot = rs_hi ? rs[1] : rs[0];
-        if (__builtin_amdgcn_ballot_w64(!(tot <= kRowSumLimit))) {
+        if (kFirst || __builtin_amdgcn_ballot_w64(!(tot <= kRowSumLimit))) {
             float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
 #pragma unroll
             for (int v = 3; v < 31; v += 2) mx = fmaxf(fmaxf(mx, s[v]), s[v + 1]);
@@ -1168,7 +1187,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             gd_next = load_gd(2);
         }
         __builtin_amdgcn_s_waitcnt(0);
-        for (int t = 0; t < ntiles; ++t) {
+        auto step = [&](auto first, int t) __attribute__((always_inline)) {
             unsigned char* kcur = k_lds + (t & 1) * kBf16TileBytes;
             // V of step t - 1 (pending product); step t + 2's goes there next
             unsigned char* vprev = v_lds + v_of(v3, 2);
@@ -1182,7 +1201,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             wait_vm<1>();
             wg_barrier();
             if (active) {
-                compute_tile(tix(t), kcur, vprev, [&](int ks) {
+                compute_tile(first, tix(t), kcur, vprev, [&](int ks) {
                     if ((ks & 1) == 0) copy_gd(ks >> 1);
                 }, [] {});
             } else {
@@ -1195,7 +1214,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             kv_next = next_off(kv_next, t + 2, kv_step, kv_wrap);
             gd_key = next_off(gd_key, t + 2, key_step, key_wrap);
             gd_next = load_gd(t + 3);
-        }
+        };
+        if (first_apart && ntiles > 0) step(std::true_type{}, 0);
+        for (int t = first_apart; t < ntiles; ++t) step(std::false_type{}, t);
     } else {
         if (ntiles > 0) {
             const unsigned hw0 = load_map(0, key_first);
@@ -1211,7 +1232,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
         // Compiler-visible wait for every load so far (Q, map, tile 0): the
         // loop then never waits for vector memory on the Q registers' account.
         __builtin_amdgcn_s_waitcnt(0);
-        for (int t = 0; t < ntiles; ++t) {
+        auto step = [&](auto first, int t) __attribute__((always_inline)) {
             // t counts loop steps; step t computes tile tix(t). Step t's K tile
             // lives in stage t & 1, its V tile in stage t % 3; step t+1's
             // tile streams into the next stage, which held a tile that every
@@ -1248,7 +1269,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             };
             if (active) {
                 compute_tile(
-                    tix(t), kcur, v_lds + v_of(v3, 2),
+                    first, tix(t), kcur, v_lds + v_of(v3, 2),
                     [&](int ks) {
                         if ((ks & 1) == 0) copy_plain(ks >> 1);
                     },
@@ -1259,7 +1280,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
                 overwrite();
             }
             v3 = v_next(v3);
-        }
+        };
+        if (first_apart && ntiles > 0) step(std::true_type{}, 0);
+        for (int t = first_apart; t < ntiles; ++t) step(std::false_type{}, t);
     }
     if (active && ntiles > 0) pv_last(v_lds + v_of(v3, 2));
     // the trailing copies land before the workgroup's LDS is released, and

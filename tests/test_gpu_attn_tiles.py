@@ -65,3 +65,10 @@ def test_tile_counts(keys, scale):
     vb[rows.to(DEV)] = float("nan")
     via_map = _run(q, kb, vb, heads, arena.to(DEV), kvmap.to(DEV))
     assert torch.equal(via_map, got)
+
+
+@pytest.mark.parametrize("keys", [1023, 1024, 1025, 1089])
+def test_tile_counts_around_a_short_walk(keys):
+    """Without a map, walks of up to 16 tiles start with a step of their own and
+    longer ones with a product of zeros; with one, all start with the former."""
+    test_tile_counts(keys, 4.0)
