@@ -838,12 +838,14 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     // third of its time. Its only independent work is the tile before:
     // MFMA + FMA + exponential + pack interleaved take 35 cycles, the MFMA
     // alone 32.5, so the scheduling barriers keep the order written here.
-    // Before -> after (PV under its own tile's step -> under the next): 21
-    // causal frames x 3600 tokens, 12 heads, 16.79 -> 15.07 ms (1.22 PFLOP/s,
-    // the rate of a large library bf16 product on the same card); 8 frames
-    // within themselves, 1560 tokens, 131 -> 126 us; 8 causal steps through
-    // the map 689 -> 648 us. Waves of 64 queries, one per SIMD, on the same
-    // schedule: 16.3 ms and 153 us.
+    // Before -> after (PV under its own tile's step -> under the next), both in
+    // turn on one card: 21 causal frames x 3600 tokens, 12 heads, 16.16 -> 14.64
+    // ms (1.26 PFLOP/s; a large library bf16 product runs at 1.39 there); 8 frames
+    // within themselves, 1560 tokens, 129 -> 125 us; 8 causal steps through the map
+    // 678 -> 636 us. (On hotter cards 17.1 -> 15.2 and 16.9 -> 15.6 ms.) Only 4
+    // frames of 1560 tokens within themselves, 1.2 rounds of workgroups, lost: 76.5
+    // -> 79 us. Waves of 64 queries, one per SIMD, on the same schedule: 16.3 ms
+    // and 153 us where this took 15.1 and 126.
     // The values and the order in which they are added to O are those of the
     // product taken in the tile's own step. The first step has no product
     // pending and no running max to exponentiate against; it is a step of its
@@ -1260,6 +1262,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             // wave-uniform: the group mixes arena and original rows. Its arena
             // rows go out after the copies of the original ones and replace
             // them (a wave's vector-memory operations complete in issue order).
+            // That reads up to twice the rows, and maps scattered row by row do
+            // not lose by it: 1560 queries on 12480 keys, half of them in the
+            // arena, took 163 us before this and the deferred product, and take
+            // 151; a tenth of them 157 and 140.
             const bool mixed = kMap && grp_mapped && !(kRuns && grp_run);
             auto overwrite = [&] {
                 if (__builtin_expect(!mixed, 1)) return;

@@ -8,7 +8,7 @@
 // The algorithm is the one OpenCV 4.x publishes (modules/video/src/
 // optflowgf.cpp; Farneback, "Two-frame motion estimation based on
 // polynomial expansion", SCIA 2003), laid out for the GPU: a launch covers many
-// frames (or consecutive pairs) of a clip, the pyramid kernels several levels,
+// frames (or consecutive pairs: chunk_pairs) of a clip, the pyramid kernels several levels,
 // and each frame's pyramid image and polynomial expansion are computed once per
 // level and shared by the two pairs that use it.
 //
@@ -171,7 +171,7 @@ __device__ __forceinline__ const PyrLevel& pyr_level(const PyrArgs& a, int block
 // (rows) are neighbours and share their taps' reads. Nothing but the uint8
 // source is read from HBM and nothing but the level is written: as two launches
 // per level with the x-blurred rows in HBM the three reduced levels of a
-// 50-frame 832x480 clip took 249 us, and take 155 us in one launch for all of them
+// 50-frame 832x480 clip took 247 us, and take 148 us in one launch for all of them
 // (bound by the taps' byte reads and conversions on the VALU).
 template <int kTaps>
 __device__ __forceinline__ void preblur_tile(const PyrArgs& a, const PyrLevel& L, float* hb) {
@@ -674,9 +674,9 @@ __global__ __launch_bounds__(256) void update_matrices_kernel(FlowArgs a, float*
 // Two LDS buffers, so that a batch's samples need not wait for the last
 // batch's solves.
 //
-// Bound by the L1's gather rate and the VALU rather than by memory: 5.4 us an
-// iteration and pair of 832x480, where matrix update and box filter launches
-// took 8.1 us.
+// Bound by the L1's gather rate and the VALU rather than by memory: 5.0 us an
+// iteration and pair of 832x480 in a 50-frame clip, where matrix update and box
+// filter launches took 8.3 us.
 // kZero: the current flow is zero (the first iteration of the coarsest level).
 template <bool kZero>
 __global__ __launch_bounds__(kFsThreads, 4) void flow_step_kernel(FlowArgs a) {

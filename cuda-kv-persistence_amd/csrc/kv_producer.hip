@@ -13,7 +13,8 @@
 //                       the values are this library's own, not torch's.
 //   linear()            y = x W^T + b (+ y) (nn.Linear, backbone.py:13-14,44):
 //                       the grouped projection kernel where it tiles the
-//                       shape, else the generic fp32-matrix-core kernel
+//                       shape, fp32 layers of at most 16 inputs on a kernel
+//                       of their own, else the generic fp32-matrix-core kernel
 //                       (proj_gemm.hip); out_proj adds into the residual
 //                       stream in the epilogue.
 //   Backbone            token_embed -> blocks -> final_norm (backbone.py:58-67);
@@ -203,9 +204,10 @@ int launch_ok(const char* what) {
 // ---------------------------------------------------------------------------
 // Linear layers: the grouped projection kernel for the shapes it tiles (K a
 // multiple of 128 bytes, N % 128, 16-byte aligned operands: every projection
-// of the reference's configuration, in both precisions), the generic
+// of the reference's configuration, in both precisions), the short-inner kernel
+// for fp32 layers of 4, 8, 12 or 16 inputs that are large enough, the generic
 // fp32-matrix-core kernel for every other shape (proj_gemm.hip). In fp32 the
-// LayerNorm and three 1560 x 1536 x 1536 projections take 187 us tiled and 696
+// LayerNorm and three 1560 x 1536 x 1536 projections take 187 us tiled and 687
 // us generic. No library GEMM.
 // ---------------------------------------------------------------------------
 

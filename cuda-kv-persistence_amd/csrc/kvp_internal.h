@@ -114,14 +114,15 @@ int fill_words(void* dst, long n, unsigned value, void* stream);
 // outs[g][r, n] = sum_k x[r, k] w[g*Ng + n, k] + bias[g*Ng + n]
 // (+ outs[g][r, n] when accumulate; fp32 output only). x, w of in_dtype (0 =
 // fp32, 1 = bf16); bias fp32 or null; out_dtype 0 = fp32, 1 = bf16 (fp32
-// operands: fp32 only); tile_n 128 (the tiles measured fastest for the
-// shape) or 256 (bf16 operands: 256 x 256 tiles).
+// operands: fp32 only); tile_n 128 (tiles chosen by size: choose_tile) or 256
+// (bf16 operands: 256 x 256 tiles).
 // Returns 0 on success, 2 when the shape is outside the kernel's tiling
 // (K % 64, fp32 K % 32, or Ng % tile_n), 1 on any other error.
 int launch_proj_gemm(int in_dtype, const void* x, const void* w, const float* bias,
                      void* const* outs, int groups, long rows, int K, int Ng, int out_dtype,
                      bool accumulate, int tile_n, void* stream);
-// Any-shape linear layer (proj_gemm.hip, fp32 matrix cores):
+// Any-shape linear layer (proj_gemm.hip, fp32 matrix cores; fp32 layers of 4, 8,
+// 12 or 16 inputs that are large enough on plain fp32 FMAs):
 // y[r, n] = sum_k x[r, k] w[n, k] + bias[n] (+ y[r, n] when accumulate, fp32
 // output only); in/out dtype pairs fp32->fp32, bf16->bf16, bf16->fp32.
 int launch_gemm_generic(int in_dtype, int out_dtype, const void* x, const void* w,

@@ -124,9 +124,12 @@ __device__ __forceinline__ int pj_xcd_remap(int bid, int n) {
 // fp32 (q/k/v of one frame, 1560 rows, K = 1536, 3 x 1536 features) is bound by
 // the fp32 matrix cores (157 TFLOP/s peak): LayerNorm and this launch take
 // 187 us, 123 TFLOP/s in the GEMM; three launches of the bounds-checked
-// any-shape kernel below took 696 us with the same LayerNorm. A chunk's 64
+// any-shape kernel below took 687-696 us with the same LayerNorm. A chunk's 64
 // MFMAs per wave (4,096 cycles) cover its copies many times over. 468
-// workgroups on 512 slots leave 9 % of the chip idle.
+// workgroups on 512 slots leave 9 % of the chip idle. One size for all: a single
+// layer of few rows is one wave per SIMD of a few CUs, its time the chain of
+// chunks (16 rows x 1536 -> 1536: 101 us; 224 any-shape with the weights from
+// HBM, 92 with the same weights in the L2 call after call).
 template <typename InT, int TN, int TR, typename OutT, bool kAcc>
 __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_small_kernel(ProjArgs a) {
     constexpr int JN = TN / 64, JR = TR / 64;
@@ -362,14 +365,16 @@ __global__ __launch_bounds__(kPThreads, 2) void proj_gemm_small_kernel(ProjArgs 
 // 256 x 320 draws less than half the L2 bytes per MFMA of a 128 x 128 one. The
 // chunk barrier sits between the last k-step's MFMAs, so that the next chunk's
 // first fragments arrive under the rest of them, and the copies of a chunk
-// (2.5 us of MFMAs ahead of their use) are spread over the k-steps.
+// (a chunk's MFMAs, 2,560 cycles per SIMD or about 1 us, ahead of their use) are
+// spread over the k-steps.
 // A tile may hold features of two groups (each wave's 64 lie in one) and reach
 // past the last group.
 //
-// 12,480 tokens, K = 1536: q/k/v 3 x 1536 features in 153 us (1,151 TFLOP/s;
-// 128 x 128 tiles: 205 us on the same GPU), out_proj + residual in 69 us (85).
-// Beyond the MFMAs a tile's epilogue and first chunk are exposed, with one
-// workgroup per CU.
+// 12,480 tokens, K = 1536, kernel times within a backbone's forward: q/k/v, 3 x
+// 1536 features, 145 us (1,217 TFLOP/s; 128 x 128 tiles 169 us on the same card),
+// out_proj + residual 68 us (82). Called back to back the card's power sets the
+// rate: choose_tile. Beyond the MFMAs a tile's epilogue and first chunk are
+// exposed, with one workgroup per CU.
 template <int JR, typename OutT, bool kAcc>
 __global__ __launch_bounds__(kWThreads, 2) void proj_gemm_wide_kernel(ProjArgs a) {
     constexpr int TN = kWTileN, TR = 64 * JR, JN = 2;
@@ -818,8 +823,9 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GenericArgs a) {
 // walks kThinRows rows, whose values are wave-uniform (scalar loads), so a row
 // costs 4 K FMAs and one 16-byte store per lane: bound by writing y. The
 // 64 x 64 tiles of gemm_generic_kernel pad K to 32 and stage both operands
-// through LDS for one chunk of work. 12480 rows x 16 -> 1536 features:
-// 51 -> 32 us (2.4 TB/s written). 8 rows per wave 32.6 us, 32 rows 38.7.
+// through LDS for one chunk of work. 12480 rows x 16 -> 1536 features, within a
+// backbone's forward: 46 -> 28 us (2.8 TB/s written; with 16 rows per wave 32 us,
+// 8 rows took 32.6 and 32 rows 38.7).
 // short_inner says where it is used.
 constexpr int kThinRows = 16;
 constexpr int kThinCols = 256;

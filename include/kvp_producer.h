@@ -35,8 +35,10 @@ int kvp_layer_norm(int in_dtype, int out_dtype, const void* x,
  * fp32 output only). W has the storage dtype of x; bias fp32 [out] or NULL.
  * (in_dtype, out_dtype): (0, 0), (1, 1) or (1, 0). Any shape: shapes
  * with in % 64 == 0 (fp32: in % 32 == 0), out % 128 == 0 and 16-byte aligned
- * operands run on the tiled projection kernels (see kvp_proj_gemm), every other
- * shape on this library's generic fp32-matrix-core kernel; no library GEMM. */
+ * operands run on the tiled projection kernels (see kvp_proj_gemm), fp32 layers
+ * with in = 4, 8, 12 or 16, out % 4 == 0 and aligned weights, bias and output that
+ * are large enough on a kernel of plain fp32 FMAs, every other shape on this
+ * library's generic fp32-matrix-core kernel; no library GEMM. */
 int kvp_linear(int in_dtype, int out_dtype, const void* x, const void* w,
                const float* bias, void* y, long rows, int in_features,
                int out_features, int accumulate, void* stream);
@@ -57,8 +59,8 @@ int kvp_linear_kernel(int in_dtype, int out_dtype, long rows, int in_features,
  * all groups: the q/k/v row blocks of qkv_proj written to three outputs, or
  * out_proj added into the fp32 residual stream (reference:
  * src/backbone.py:13-14,18-22,32-33). K a multiple of 64, N a multiple of
- * tile_n: 128 = the tiles measured fastest for the shape (128 x 128 or 256
- * features x 256 or 320 tokens); 256 = 256 x 256 tiles. The results are the
+ * tile_n: 128 = 128 x 128 tiles or 256 features x 256 or 320 tokens, chosen by
+ * the shape (kvp_linear_kernel); 256 = 256 x 256 tiles. The results are the
  * same bit for bit. Unused outputs may be NULL. */
 int kvp_proj_gemm(const void* x, const void* w, const float* bias,
                   void* out0, void* out1, void* out2, int groups, long rows,
