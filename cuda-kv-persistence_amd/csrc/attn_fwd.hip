@@ -76,6 +76,7 @@ constexpr int kNumXcd = 8;
 constexpr float kLog2e = 1.4426950408889634f;
 
 constexpr int kBf16BlockKeys = 64;
+constexpr int kShortWalk = 16;  // most tiles of a map-free walk whose first step is apart
 constexpr int kF32BlockKeys = 32;
 
 struct AttnArgs {
@@ -488,9 +489,11 @@ __device__ __forceinline__ void store_rows_staged(const AttnArgs& a, const WgCoo
 // kGd (KVMap launches with group descriptors, a.gdesc): each wave reads its
 // copy group's 8-byte descriptor per tile instead of the group's 16 map
 // entries; only groups whose descriptor says "general" read the entries.
-template <typename OutT, bool kMap, bool kColdNt, bool kCyclic, bool kGd = false>
+template <typename OutT, bool kMap, bool kColdNt, bool kCyclic, bool kGd = false,
+          bool kShort = false>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) {
     static_assert(!kGd || (kMap && !kColdNt), "group descriptors serve the KVMap kernel");
+    static_assert(!kShort || (!kMap && !kCyclic), "short walks: map-free, without a window");
     constexpr int kColdAux = kColdNt ? 2 : 0;  // buffer-load aux: bit 1 = nt
     // K in a ring of two stages, V in three: a tile's PV product runs under the
     // next tile's softmax, so its V stays for one more step.
@@ -850,14 +853,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
     // product taken in the tile's own step. The first step has no product
     // pending and no running max to exponentiate against; it is a step of its
     // own (kFirst) that leaves both out: key ranges of one tile 5.3 -> 4.5 us, 50
-    // frames of 900 tokens within themselves 295 -> 288. But without a map, walks
-    // of more than kShortWalk tiles gain less than their workgroups lose by
-    // starting in step (8 frames of 1560 tokens 126.4 -> 128.4): there the first
-    // step's pending product is 0 x 0.
-    constexpr int kShortWalk = 16;
-    const bool first_apart = kMap || ntiles <= kShortWalk;
+    // frames of 900 tokens within themselves 295 -> 288. But without a map, long
+    // walks gain less than their workgroups lose by starting so (8 frames of 1560
+    // tokens 125.3 -> 127.7 us, 21 causal frames of 3600 unchanged): there (kShort
+    // false) the first step's pending product is 0 x 0.
+    constexpr bool kFirstApart = kMap || kShort;
     u32x4 pd[4];
-    if (!first_apart) {
+    if constexpr (!kFirstApart) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) pd[g] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
@@ -1217,8 +1219,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             gd_key = next_off(gd_key, t + 2, key_step, key_wrap);
             gd_next = load_gd(t + 3);
         };
-        if (first_apart && ntiles > 0) step(std::true_type{}, 0);
-        for (int t = first_apart; t < ntiles; ++t) step(std::false_type{}, t);
+        if (kFirstApart && ntiles > 0) step(std::bool_constant<kFirstApart>{}, 0);
+        for (int t = kFirstApart; t < ntiles; ++t) step(std::false_type{}, t);
     } else {
         if (ntiles > 0) {
             const unsigned hw0 = load_map(0, key_first);
@@ -1287,8 +1289,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_bf16_kernel(AttnArgs a) 
             }
             v3 = v_next(v3);
         };
-        if (first_apart && ntiles > 0) step(std::true_type{}, 0);
-        for (int t = first_apart; t < ntiles; ++t) step(std::false_type{}, t);
+        if (kFirstApart && ntiles > 0) step(std::bool_constant<kFirstApart>{}, 0);
+        for (int t = kFirstApart; t < ntiles; ++t) step(std::false_type{}, t);
     }
     if (active && ntiles > 0) pv_last(v_lds + v_of(v3, 2));
     // the trailing copies land before the workgroup's LDS is released, and
@@ -2077,6 +2079,9 @@ int launch_attention(const AttnLaunch& L) {
                                dim3((unsigned)p.grid), dim3(kThreads), 0, st, a);
         else if (a.cyclic)
             hipLaunchKernelGGL((attn_fwd_bf16_kernel<__bf16, false, false, true>),
+                               dim3((unsigned)p.grid), dim3(kThreads), 0, st, a);
+        else if (p.keys_per_split <= kShortWalk * kBf16BlockKeys)
+            hipLaunchKernelGGL((attn_fwd_bf16_kernel<__bf16, false, false, false, false, true>),
                                dim3((unsigned)p.grid), dim3(kThreads), 0, st, a);
         else
             hipLaunchKernelGGL((attn_fwd_bf16_kernel<__bf16, false, false, false>),

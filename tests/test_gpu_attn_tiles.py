@@ -69,6 +69,6 @@ def test_tile_counts(keys, scale):
 
 @pytest.mark.parametrize("keys", [1023, 1024, 1025, 1089])
 def test_tile_counts_around_a_short_walk(keys):
-    """Without a map, walks of up to 16 tiles start with a step of their own and
-    longer ones with a product of zeros; with one, all start with the former."""
+    """Without a map, walks of up to 16 tiles run a kernel whose first step is one of
+    its own, longer ones start with a product of zeros; with one, all do the former."""
     test_tile_counts(keys, 4.0)
