@@ -168,8 +168,10 @@ def test_fp32_qkv_project_is_three_linears(rows, heads):
         assert torch.equal(got, want), i
 
 
-# the wide tiles: tokens that end inside a tile of 320 or 256, feature tiles that
-# hold two groups and reach past the last one, one and several K chunks
+# tokens that end inside a tile of 320, 256 or 128, feature tiles that hold two
+# groups and reach past the last one, one and several K chunks: the wide tiles for
+# tile_n 256; so few chunks run 128 x 128 tiles for tile_n 128 (where it picks the
+# wide ones: test_chosen_wide_tiles_match_oracle)
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,K,N,groups,tile_n,out_dt,acc,bias", [
     (12473, 64, 1408, 3, 128, 1, False, True),
